@@ -556,18 +556,14 @@ __device__ __forceinline__ void update_tile(const DevGeom& g, const SlotTab& S, 
 
 // Fused OSTR update with the exact transpose (the matched counterpart of
 // update_fused_kernel): per voxel capL = M (0 + sum_views cos sum_i a_ij h_i)
-// from matched_voxel, then the prior window on x_in and the SQS update into
-// x_out, the same epilogue (update_rows). h detector-row-major. One row per
-// lane (MATCHED_ROWS = 1): the gather dominates and is latency-bound, so the
-// launch keeps as many waves as the standalone transpose.
-constexpr int MATCHED_ROWS = 1;
-
-template <int POT, typename TI, typename TP>
+// from matched_rows, then the prior window on x_in and the SQS update into
+// x_out, the same epilogue (update_rows). h detector-row-major. R rows per
+// lane (matched_row_count).
+template <int POT, typename TI, typename TP, int R>
 __global__ __launch_bounds__(256) void update_fused_matched_kernel(
     DevGeom g, MatchedSlots S, int n_slots, const TP* __restrict__ hsub,
     const TI* __restrict__ x_in, TI* __restrict__ x_out, const float* __restrict__ d,
     PriorClass W, float inv_delta, float beta, float capl_scale, int guard) {
-    constexpr int R = MATCHED_ROWS;
     const TileCoord c = tile_coord<R, CASE_WAVES>(g, xcd_tile(blockIdx.x, gridDim.x));
     if (c.iy0 >= g.ny) return;  // see sbp_kernel
     const uint32_t nvox = (uint32_t)g.nx * g.ny * g.nz;
@@ -576,11 +572,7 @@ __global__ __launch_bounds__(256) void update_fused_matched_kernel(
     const VolWriter<TI> XO(x_out, nvox);
     const VolReader<float> D(d, nvox);
     float total[R];
-#pragma unroll
-    for (int r = 0; r < R; ++r)
-        total[r] = (c.ix < g.nx && c.iy0 + r < g.ny)
-                       ? matched_voxel<TP>(g, S, n_slots, 1, P, c.ix, c.iy0 + r, c.iz)
-                       : 0.0f;
+    matched_rows<TP, R>(g, S, n_slots, 1, P, c.ix, c.iy0, c.iz, total);
     by_prior_mode<R>(g, c, W, [&](auto m) {
         update_rows<POT, decltype(m)::value, TI, R>(g, X, XO, D, c, total, W, inv_delta,
                                                     beta, capl_scale, guard);
@@ -830,16 +822,34 @@ hipError_t launch_sart_update_fused(const DevGeom& g, const ViewTab* views, int 
 
 namespace {
 
+template <int POT, typename TI, typename TP, int R>
+hipError_t fused_matched_r(const DevGeom& g, const MatchedSlots& S, int n, const void* x_in,
+                           void* x_out, const float* d, const void* hsub, const PriorClass& W,
+                           float inv_delta, float beta, float capl_scale, int guard,
+                           hipStream_t st) {
+    const dim3 grid(volume_tiles(g, R * CASE_WAVES));
+    hipLaunchKernelGGL((update_fused_matched_kernel<POT, TI, TP, R>), grid, dim3(256), 0, st, g,
+                       S, n, (const TP*)hsub, (const TI*)x_in, (TI*)x_out, d, W, inv_delta, beta,
+                       capl_scale, guard);
+    return hipGetLastError();
+}
+
 template <int POT, typename TI, typename TP>
 hipError_t fused_matched_t(const DevGeom& g, const MatchedSlots& S, int n, const void* x_in,
                            void* x_out, const float* d, const void* hsub, const PriorClass& W,
                            float inv_delta, float beta, float capl_scale, int guard,
                            hipStream_t st) {
-    const dim3 grid(volume_tiles(g, MATCHED_ROWS * CASE_WAVES));
-    hipLaunchKernelGGL((update_fused_matched_kernel<POT, TI, TP>), grid, dim3(256), 0, st, g, S,
-                       n, (const TP*)hsub, (const TI*)x_in, (TI*)x_out, d, W, inv_delta, beta,
-                       capl_scale, guard);
-    return hipGetLastError();
+    switch (matched_row_count(g)) {
+        case 4:
+            return fused_matched_r<POT, TI, TP, 4>(g, S, n, x_in, x_out, d, hsub, W, inv_delta,
+                                                   beta, capl_scale, guard, st);
+        case 2:
+            return fused_matched_r<POT, TI, TP, 2>(g, S, n, x_in, x_out, d, hsub, W, inv_delta,
+                                                   beta, capl_scale, guard, st);
+        default:
+            return fused_matched_r<POT, TI, TP, 1>(g, S, n, x_in, x_out, d, hsub, W, inv_delta,
+                                                   beta, capl_scale, guard, st);
+    }
 }
 
 template <int POT, typename TI>
@@ -891,12 +901,7 @@ hipError_t launch_update_fused_matched(const DevGeom& g, const ViewTab* views, i
                                        float beta, float capl_scale, int potential, float delta,
                                        float rho, int guard, hipStream_t st) {
     if (a1 - a0 > MAX_SLOTS || a1 < a0) return hipErrorInvalidValue;
-    MatchedSlots S;
-    for (int a = a0; a < a1; ++a) {
-        S.x0[a - a0] = views[a].x0;
-        S.z0[a - a0] = views[a].z0;
-        S.c[a - a0] = views[a].c;
-    }
+    const MatchedSlots S = matched_slots(g, views + a0, a1 - a0);
     PriorW W27;
     prior_weights(W27.w, rho);
     const PriorClass W = prior_params(W27, potential, delta);

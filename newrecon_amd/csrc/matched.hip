@@ -2,7 +2,7 @@
 //
 // No reference counterpart: the reference backprojects with the unmatched
 // bilinear SBP (Tomo_OSTR.cu:1553-1734). This kernel accumulates, for every
-// voxel j, x_j += sum_views cos(t) sum_i a_ij p_i (matched_voxel in
+// voxel j, x_j += sum_views cos(t) sum_i a_ij p_i (matched_rows in
 // matched_device.h: the candidate bins of the voxel's shadow, each ray clipped
 // against the voxel box).
 #include "matched_device.h"
@@ -11,31 +11,49 @@ namespace ostr {
 
 namespace {
 
-// One voxel per lane: 64 lanes on consecutive voxels along x, one row per
-// wave (4 rows per work-group), one slice per grid z. Deterministic: every
-// voxel is owned by one lane, no atomics.
-template <typename TP>
+// 64 lanes on consecutive voxels along x, R rows per wave (4 waves per
+// work-group), one slice. Deterministic: every voxel is owned by one lane, no
+// atomics.
+template <typename TP, int R>
 __global__ __launch_bounds__(256) void matched_kernel(DevGeom g, MatchedSlots S, int n_slots,
                                                       int cos_weight,
                                                       const TP* __restrict__ prj,
                                                       float* __restrict__ img) {
-    const int ix = blockIdx.x * 64 + (threadIdx.x & 63);
-    const int iy = blockIdx.y * 4 + (threadIdx.x >> 6);
-    const int iz = blockIdx.z;
-    if (ix >= g.nx || iy >= g.ny) return;
+    const int tiles_x = (g.nx + 63) / 64, tiles_y = (g.ny + 4 * R - 1) / (4 * R);
+    const int t = xcd_tile(blockIdx.x, gridDim.x);
+    const int ix = (t % tiles_x) * 64 + (threadIdx.x & 63);
+    const int iy0 = ((t / tiles_x) % tiles_y) * 4 * R + (threadIdx.x >> 6) * R;
+    const int iz = t / tiles_x / tiles_y;
+    if (iy0 >= g.ny) return;
     const VolReader<TP> P(prj, (uint32_t)n_slots * g.nbx * g.nby);
-    const float total = matched_voxel<TP>(g, S, n_slots, cos_weight, P, ix, iy, iz);
-    const int64_t vi = ((int64_t)iz * g.ny + iy) * g.nx + ix;
-    img[vi] = img[vi] + total;
+    float total[R];
+    matched_rows<TP, R>(g, S, n_slots, cos_weight, P, ix, iy0, iz, total);
+    if (ix >= g.nx) return;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        if (iy0 + r >= g.ny) break;
+        const int64_t vi = ((int64_t)iz * g.ny + iy0 + r) * g.nx + ix;
+        img[vi] = img[vi] + total[r];
+    }
+}
+
+template <typename TP, int R>
+hipError_t matched_r(const DevGeom& g, const MatchedSlots& S, int n, int cos_weight,
+                     const void* prj, float* img, hipStream_t st) {
+    const unsigned grid = (unsigned)((g.nx + 63) / 64) * ((g.ny + 4 * R - 1) / (4 * R)) * g.nz;
+    hipLaunchKernelGGL((matched_kernel<TP, R>), dim3(grid), dim3(256), 0, st, g, S, n, cos_weight,
+                       (const TP*)prj, img);
+    return hipGetLastError();
 }
 
 template <typename TP>
 hipError_t matched_t(const DevGeom& g, const MatchedSlots& S, int n, int cos_weight,
                      const void* prj, float* img, hipStream_t st) {
-    dim3 grid((g.nx + 63) / 64, (g.ny + 3) / 4, g.nz);
-    hipLaunchKernelGGL((matched_kernel<TP>), grid, dim3(256), 0, st, g, S, n, cos_weight,
-                       (const TP*)prj, img);
-    return hipGetLastError();
+    switch (matched_row_count(g)) {
+        case 4: return matched_r<TP, 4>(g, S, n, cos_weight, prj, img, st);
+        case 2: return matched_r<TP, 2>(g, S, n, cos_weight, prj, img, st);
+        default: return matched_r<TP, 1>(g, S, n, cos_weight, prj, img, st);
+    }
 }
 
 }  // namespace
@@ -45,12 +63,7 @@ hipError_t launch_matched_rows(const DevGeom& g, const ViewTab* views, int a0, i
                                int prj_dtype, hipStream_t st) {
     for (int b = a0; b < a1; b += MAX_SLOTS) {
         const int e = b + MAX_SLOTS < a1 ? b + MAX_SLOTS : a1;
-        MatchedSlots S;
-        for (int a = b; a < e; ++a) {
-            S.x0[a - b] = views[a].x0;
-            S.z0[a - b] = views[a].z0;
-            S.c[a - b] = views[a].c;
-        }
+        const MatchedSlots S = matched_slots(g, views + b, e - b);
         const size_t off = (size_t)(b - a0) * g.nbx * g.nby * elem_size(prj_dtype);
         const void* p = (const char*)prj + off;
         hipError_t err;

@@ -179,8 +179,9 @@ struct VolReader {
                                                  0x00020000);
     }
     __device__ __forceinline__ float operator()(uint32_t i) const { return at_byte(i * sizeof(T)); }
-    // the element at byte offset b (a multiple of sizeof(T))
-    __device__ __forceinline__ float at_byte(uint32_t b) const;
+    // the element at byte offset b + sb (a multiple of sizeof(T)), sb
+    // wave-uniform (the load's scalar offset)
+    __device__ __forceinline__ float at_byte(uint32_t b, uint32_t sb = 0) const;
     // elements e and e + 1 from one 8-byte load: for 4-byte types at e, for
     // 2-byte types from the 4-byte boundary at or below e, so when e is odd
     // element e + 2 must lie inside the buffer (the caller guarantees it)
@@ -192,16 +193,16 @@ struct VolReader {
                                                float& b) const;
 };
 template <>
-__device__ __forceinline__ float VolReader<float>::at_byte(uint32_t b) const {
-    return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rsrc, b, 0, 0));
+__device__ __forceinline__ float VolReader<float>::at_byte(uint32_t b, uint32_t sb) const {
+    return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rsrc, b, sb, 0));
 }
 template <>
-__device__ __forceinline__ float VolReader<bf16_t>::at_byte(uint32_t b) const {
-    return __uint_as_float((uint32_t)__builtin_amdgcn_raw_buffer_load_b16(rsrc, b, 0, 0) << 16);
+__device__ __forceinline__ float VolReader<bf16_t>::at_byte(uint32_t b, uint32_t sb) const {
+    return __uint_as_float((uint32_t)__builtin_amdgcn_raw_buffer_load_b16(rsrc, b, sb, 0) << 16);
 }
 template <>
-__device__ __forceinline__ float VolReader<_Float16>::at_byte(uint32_t b) const {
-    unsigned short h = __builtin_amdgcn_raw_buffer_load_b16(rsrc, b, 0, 0);
+__device__ __forceinline__ float VolReader<_Float16>::at_byte(uint32_t b, uint32_t sb) const {
+    unsigned short h = __builtin_amdgcn_raw_buffer_load_b16(rsrc, b, sb, 0);
     return (float)__builtin_bit_cast(_Float16, h);
 }
 typedef unsigned int u32x2_t __attribute__((ext_vector_type(2)));
