@@ -9,10 +9,9 @@
 //
 // MI355X mapping: one ray per lane, 64 lanes along detector x (the direction
 // that is contiguous in the volume, so gathers of a wave fall in a few cache
-// lines); a work-group is a 64 x 4 bin tile of one view slot; blocks of 16
-// tiles (64 x 64 bins) are dealt round-robin to the XCDs (xcd_spread_tile), so
-// each XCD gets an even share of the rays through the volume and neighbouring
-// tiles of a block share an L2.
+// lines); a work-group is a 64 x 4 bin tile of one view slot; rows of tiles of
+// all views are dealt round-robin to the XCDs (ray_tile), so each XCD gets an
+// even share of the rays through the volume and the views share its L2.
 // Per-view trig comes from the handle's table (host FP64, rounded to float).
 // The relative stop test (lmax - at)/lmax > 1e-6 is replaced by `at < thr`
 // with thr computed once per ray as the exact float boundary of that test, so
@@ -445,35 +444,39 @@ __device__ __forceinline__ void project_bin(const DevGeom& g, const ViewTab& v, 
     st<TO>(out, (KIND >= 3) ? o_row : o_ref, val);
 }
 
-// Tile t of a launch over n_slots views, TJ detector rows x 64 columns per
-// work-group; tile order: j-tile fastest, then view slot, then i-tile (the
-// groups working at one time share a view and neighbouring columns).
+// Tile counts of a detector in tiles of 64 columns x tj rows.
+__host__ __device__ __forceinline__ int ray_tiles_i(const DevGeom& g) {
+    return (g.nbx + TILE_I - 1) / TILE_I;
+}
+__host__ __device__ __forceinline__ int ray_tiles_j(const DevGeom& g, int tj) {
+    return (g.nby + tj - 1) / tj;
+}
+// Bin of this thread in tile t (TJ detector rows); false outside the detector.
 template <int TJ>
-__device__ __forceinline__ bool bin_of_tile(const DevGeom& g, int n_slots, int t, int& slot,
-                                            int& i, int& j) {
-    const int tiles_j = (g.nby + TJ - 1) / TJ;
-    const int tj = t % tiles_j;
-    const int rest = t / tiles_j;
-    slot = rest % n_slots;
-    const int ti = rest / n_slots;
-    i = ti * TILE_I + (threadIdx.x & 63);
-    j = tj * TJ + (threadIdx.x >> 6);
+__device__ __forceinline__ bool bin_of_tile(const DevGeom& g, const RayTile& t, int& i, int& j) {
+    i = t.ti * TILE_I + (threadIdx.x & 63);
+    j = t.tj * TJ + (threadIdx.x >> 6);
     return i < g.nbx && j < g.nby;
+}
+// Bin of this thread of a single-geometry launch of ray_grid() work-groups.
+__device__ __forceinline__ bool bin_of_group(const DevGeom& g, int n_slots, int& slot, int& i,
+                                             int& j) {
+    RayTile t;
+    if (!ray_tile(blockIdx.x, n_slots, ray_tiles_i(g), ray_tiles_j(g, TILE_J), t)) return false;
+    slot = t.slot;
+    return bin_of_tile<TILE_J>(g, t, i, j);
 }
 
 template <int KIND, typename TI, typename TO>
 __global__ __launch_bounds__(256) void project_kernel(DevGeom g, const ViewTab* __restrict__ views,
-                                                      int a0, int n_slots, int tiles_i,
-                                                      int tiles_j, int cos_weight,
+                                                      int a0, int n_slots, int cos_weight,
                                                       const TI* __restrict__ img,
                                                       TO* __restrict__ out,
                                                       const float* __restrict__ y,
                                                       const float* __restrict__ b,
                                                       const float* __restrict__ r) {
     int slot, i, j;
-    if (!bin_of_tile<TILE_J>(g, n_slots, xcd_spread_tile(blockIdx.x, gridDim.x), slot, i,
-                             j))
-        return;
+    if (!bin_of_group(g, n_slots, slot, i, j)) return;
     project_bin<KIND, TI, TO>(g, views[a0 + slot], slot, i, j, cos_weight, img, out, y, b, r);
 }
 
@@ -495,9 +498,7 @@ __global__ __launch_bounds__(256) void sart_project_kernel(DevGeom g,
                                                            float* __restrict__ norm,
                                                            const float* __restrict__ p_rows) {
     int slot, i, j;
-    if (!bin_of_tile<TILE_J>(g, n_slots, xcd_spread_tile(blockIdx.x, gridDim.x), slot, i,
-                             j))
-        return;
+    if (!bin_of_group(g, n_slots, slot, i, j)) return;
     const ViewTab v = views[a0 + slot];
     const float ex = bin_centre(g.x_d0, i, g.dbx);
     const float ey = bin_centre(g.y_d0, j, g.dby);
@@ -540,12 +541,9 @@ __global__ __launch_bounds__(256) void project_4r_kernel(DevGeom g,
                                                          float* __restrict__ prj4) {
     __shared__ float sub[4][64];
     const int nbx2 = 2 * g.nbx, nby2 = 2 * g.nby;
-    const int tiles_j = (nby2 + 3) / 4;
-    const int t = xcd_spread_tile(blockIdx.x, gridDim.x);
-    const int tj = t % tiles_j;
-    const int rest = t / tiles_j;
-    const int slot = rest % n_slots;
-    const int ti = rest / n_slots;
+    RayTile t;
+    if (!ray_tile(blockIdx.x, n_slots, (nbx2 + 63) / 64, (nby2 + 3) / 4, t)) return;
+    const int slot = t.slot, ti = t.ti, tj = t.tj;
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int ii = ti * 64 + lane, jj = tj * 4 + w;
     float val = 0.0f;
@@ -588,11 +586,10 @@ __global__ __launch_bounds__(64 * TJ) void batch_project_kernel(
         const BatchCase& bc = cases[c];
         const DevGeom g = uniform_copy(bc.g);
         const int n_slots = __builtin_amdgcn_readfirstlane(bc.n_slots);
-        // this XCD's contiguous share of the case's tiles, spread over the
-        // detector (only the shadow's rays walk)
-        const int n_tiles = ((g.nbx + TILE_I - 1) / TILE_I) * ((g.nby + TJ - 1) / TJ) * n_slots;
-        int slot, i, j;
-        const bool in = bin_of_tile<TJ>(g, n_slots, spread_block_perm(t, n_tiles), slot, i, j);
+        const RayTile rt = ray_tile_of_position(t, n_slots, ray_tiles_i(g), ray_tiles_j(g, TJ));
+        const int slot = rt.slot;
+        int i, j;
+        const bool in = bin_of_tile<TJ>(g, rt, i, j);
         const ViewTab v = uniform_copy(bc.v[slot]);  // slot is uniform over the group
         if (in)
             project_bin<3, TI, TO>(g, v, slot, i, j, 1, (const TI*)uniform_ptr(bc.x_in),
@@ -603,18 +600,12 @@ __global__ __launch_bounds__(64 * TJ) void batch_project_kernel(
 }
 
 __global__ __launch_bounds__(256) void count_kernel(DevGeom g, const ViewTab* __restrict__ views,
-                                                    int a0, int n_slots, int tiles_i,
-                                                    int tiles_j,
+                                                    int a0, int n_slots,
                                                     unsigned long long* __restrict__ counter) {
-    const int t = xcd_spread_tile(blockIdx.x, gridDim.x);
-    const int tj = t % tiles_j;
-    const int rest = t / tiles_j;
-    const int slot = rest % n_slots;
-    const int ti = rest / n_slots;
-    const int i = ti * TILE_I + (threadIdx.x & 63);
-    const int j = tj * TILE_J + (threadIdx.x >> 6);
+    int slot, i, j;
+    const bool in = bin_of_group(g, n_slots, slot, i, j);
     int nseg = 0;
-    if (i < g.nbx && j < g.nby) {
+    if (in) {
         const ViewTab v = views[a0 + slot];
         bool hit;
         float len;
@@ -634,13 +625,11 @@ hipError_t launch_kind(const DevGeom& g, const ViewTab* views, int a0, int a1, i
                        const void* img, void* out, const float* y, const float* b,
                        const float* r, hipStream_t st) {
     const int n_slots = a1 - a0;
-    const int tiles_i = (g.nbx + TILE_I - 1) / TILE_I;
-    const int tiles_j = (g.nby + TILE_J - 1) / TILE_J;
-    const int64_t nblocks = (int64_t)tiles_i * tiles_j * n_slots;
+    const int64_t nblocks = ray_grid(n_slots, ray_tiles_i(g), ray_tiles_j(g, TILE_J));
     if (nblocks == 0) return hipSuccess;
     if (nblocks > 0x7fffffff) return hipErrorInvalidValue;
     hipLaunchKernelGGL((project_kernel<KIND, TI, TO>), dim3((unsigned)nblocks), dim3(256), 0, st,
-                       g, views, a0, n_slots, tiles_i, tiles_j, cos_weight,
+                       g, views, a0, n_slots, cos_weight,
                        (const TI*)img, (TO*)out, y, b, r);
     return hipGetLastError();
 }
@@ -743,8 +732,7 @@ hipError_t launch_sart_project(const DevGeom& g, const ViewTab* views, int a0, i
                                int cos_weight, const float* img, float* prj, float* norm,
                                hipStream_t st) {
     const int n_slots = a1 - a0;
-    const int64_t nblocks = (int64_t)((g.nbx + TILE_I - 1) / TILE_I) *
-                            ((g.nby + TILE_J - 1) / TILE_J) * n_slots;
+    const int64_t nblocks = ray_grid(n_slots, ray_tiles_i(g), ray_tiles_j(g, TILE_J));
     if (nblocks == 0) return hipSuccess;
     if (nblocks > 0x7fffffff) return hipErrorInvalidValue;
     hipLaunchKernelGGL(sart_project_kernel<false>, dim3((unsigned)nblocks), dim3(256), 0, st, g,
@@ -756,8 +744,7 @@ hipError_t launch_sart_project_diff(const DevGeom& g, const ViewTab* views, int 
                                     int cos_weight, const float* img, const float* p_rows,
                                     float* diff_rows, hipStream_t st) {
     const int n_slots = a1 - a0;
-    const int64_t nblocks = (int64_t)((g.nbx + TILE_I - 1) / TILE_I) *
-                            ((g.nby + TILE_J - 1) / TILE_J) * n_slots;
+    const int64_t nblocks = ray_grid(n_slots, ray_tiles_i(g), ray_tiles_j(g, TILE_J));
     if (nblocks == 0) return hipSuccess;
     if (nblocks > 0x7fffffff) return hipErrorInvalidValue;
     hipLaunchKernelGGL(sart_project_kernel<true>, dim3((unsigned)nblocks), dim3(256), 0, st, g,
@@ -768,7 +755,7 @@ hipError_t launch_sart_project_diff(const DevGeom& g, const ViewTab* views, int 
 hipError_t launch_project_4r(const DevGeom& g, const ViewTab* views, int a0, int a1,
                              const float* img, float* prj, float* prj4, hipStream_t st) {
     const int n_slots = a1 - a0;
-    const int64_t nblocks = (int64_t)((2 * g.nbx + 63) / 64) * ((2 * g.nby + 3) / 4) * n_slots;
+    const int64_t nblocks = ray_grid(n_slots, (2 * g.nbx + 63) / 64, (2 * g.nby + 3) / 4);
     if (nblocks == 0) return hipSuccess;
     if (nblocks > 0x7fffffff) return hipErrorInvalidValue;
     hipLaunchKernelGGL(project_4r_kernel, dim3((unsigned)nblocks), dim3(256), 0, st, g, views,
@@ -779,12 +766,11 @@ hipError_t launch_project_4r(const DevGeom& g, const ViewTab* views, int a0, int
 hipError_t launch_count_nnz(const DevGeom& g, const ViewTab* views, int a0, int a1,
                             unsigned long long* counter, hipStream_t st) {
     const int n_slots = a1 - a0;
-    const int tiles_i = (g.nbx + TILE_I - 1) / TILE_I;
-    const int tiles_j = (g.nby + TILE_J - 1) / TILE_J;
-    const int64_t nblocks = (int64_t)tiles_i * tiles_j * n_slots;
+    const int64_t nblocks = ray_grid(n_slots, ray_tiles_i(g), ray_tiles_j(g, TILE_J));
     if (nblocks == 0) return hipSuccess;
+    if (nblocks > 0x7fffffff) return hipErrorInvalidValue;
     hipLaunchKernelGGL(count_kernel, dim3((unsigned)nblocks), dim3(256), 0, st, g, views, a0,
-                       n_slots, tiles_i, tiles_j, counter);
+                       n_slots, counter);
     return hipGetLastError();
 }
 
