@@ -37,23 +37,17 @@ __global__ __launch_bounds__(256) void matched_kernel(DevGeom g, MatchedSlots S,
     }
 }
 
-template <typename TP, int R>
-hipError_t matched_r(const DevGeom& g, const MatchedSlots& S, int n, int cos_weight,
-                     const void* prj, float* img, hipStream_t st) {
-    const unsigned grid = (unsigned)((g.nx + 63) / 64) * ((g.ny + 4 * R - 1) / (4 * R)) * g.nz;
-    hipLaunchKernelGGL((matched_kernel<TP, R>), dim3(grid), dim3(256), 0, st, g, S, n, cos_weight,
-                       (const TP*)prj, img);
-    return hipGetLastError();
-}
-
 template <typename TP>
 hipError_t matched_t(const DevGeom& g, const MatchedSlots& S, int n, int cos_weight,
                      const void* prj, float* img, hipStream_t st) {
-    switch (matched_row_count(g)) {
-        case 4: return matched_r<TP, 4>(g, S, n, cos_weight, prj, img, st);
-        case 2: return matched_r<TP, 2>(g, S, n, cos_weight, prj, img, st);
-        default: return matched_r<TP, 1>(g, S, n, cos_weight, prj, img, st);
-    }
+    return by_matched_rows(g, [&](auto rows) {
+        constexpr int R = decltype(rows)::value;
+        const unsigned grid =
+            (unsigned)((g.nx + 63) / 64) * ((g.ny + 4 * R - 1) / (4 * R)) * g.nz;
+        hipLaunchKernelGGL((matched_kernel<TP, R>), dim3(grid), dim3(256), 0, st, g, S, n,
+                           cos_weight, (const TP*)prj, img);
+        return hipGetLastError();
+    });
 }
 
 }  // namespace

@@ -41,12 +41,6 @@
 
 namespace ostr {
 
-// mx, my: margin of the candidate ranges in bins (matched_margin).
-struct MatchedSlots {
-    float x0[MAX_SLOTS], z0[MAX_SLOTS], c[MAX_SLOTS];
-    float mx, my;
-};
-
 // Margin in bins that covers the FP32 error of a shadow end's bin coordinate
 // along one axis: the end is s + (b - s) t with t = (ez - sz) / (bz - sz), each
 // operand within a few 2^-24 of its magnitude, t also of the cancellation in
@@ -92,6 +86,15 @@ inline MatchedSlots matched_slots(const DevGeom& g, const ViewTab* v, int n) {
 inline int matched_row_count(const DevGeom& g) {
     const int64_t waves = (int64_t)((g.nx + 63) / 64) * g.ny * g.nz;  // at R = 1
     return waves >= 16384 ? 4 : waves >= 4096 ? 2 : 1;
+}
+// f(std::integral_constant<int, R>) for the geometry's row count.
+template <typename F>
+hipError_t by_matched_rows(const DevGeom& g, F f) {
+    switch (matched_row_count(g)) {
+        case 4: return f(std::integral_constant<int, 4>());
+        case 2: return f(std::integral_constant<int, 2>());
+        default: return f(std::integral_constant<int, 1>());
+    }
 }
 
 // origin + (i + 1/2) size rounded once to float: i + 1/2 is exact in FP32

@@ -41,6 +41,13 @@ struct SlotTab {
     float num[MAX_SLOTS];  // |S|^2 evaluated as fma(z0,z0,fma(y0,y0,x0*x0))
 };
 
+// Slot parameters of the exact transpose.
+// mx, my: margin of the candidate ranges in bins (matched_margin).
+struct MatchedSlots {
+    float x0[MAX_SLOTS], z0[MAX_SLOTS], c[MAX_SLOTS];
+    float mx, my;
+};
+
 // 27-neighbour prior weights, index dz*9 + dy*3 + dx (centre 13 is 0).
 struct PriorW {
     float w[27];
@@ -82,6 +89,28 @@ inline PriorClass prior_params(const PriorW& W, int potential, float delta) {
     P.k = potential == OSTR_PRIOR_LANGE ? (float)ad : (float)(ad * ad);
     return P;
 }
+
+// A fused OSTR update: geometry, buffers, prior and scalars of one call, and its
+// launchers by image storage type (update_f32.hip, update_bf16.hip,
+// update_f16.hip): with SBP, with the exact transpose.
+struct UpdateCall {
+    DevGeom g;
+    int n_slots;
+    const void* x_in;
+    void* x_out;
+    const float* d;
+    const void* hsub;
+    int prj_dtype, potential;
+    PriorClass W;
+    float inv_delta, beta, capl_scale;
+    int guard;
+};
+hipError_t update_fused_f32(const SlotTab& S, const UpdateCall& u, hipStream_t st);
+hipError_t update_fused_bf16(const SlotTab& S, const UpdateCall& u, hipStream_t st);
+hipError_t update_fused_f16(const SlotTab& S, const UpdateCall& u, hipStream_t st);
+hipError_t update_matched_f32(const MatchedSlots& S, const UpdateCall& u, hipStream_t st);
+hipError_t update_matched_bf16(const MatchedSlots& S, const UpdateCall& u, hipStream_t st);
+hipError_t update_matched_f16(const MatchedSlots& S, const UpdateCall& u, hipStream_t st);
 
 // One case of a batched launch (device-resident table, rebuilt per call).
 struct BatchCase {
