@@ -56,3 +56,14 @@ def test_fused_sart_update(case, beta):
     prior = S.prior_sart(x, 1e-3) if beta else None
     want = S.bproj_sart(h.transpose(1, 2).contiguous(), 0, 2, x.clone(), 0.9, prior, beta)
     assert torch.equal(out, want)
+
+
+@pytest.mark.parametrize("nbx,nby,n", [(1, 1, 1), (33, 31, 2), (65, 127, 3), (700, 1300, 3)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_layout_transpose(dev, nbx, nby, n, dtype):
+    """Both tile sizes of the layout transpose (the larger from 512 tiles of
+    64x64 on), whole and ragged."""
+    g = Geometry.half_cone(4, 4, 2, 1.0, 1.0, 1.0, nbx, nby, 1.0, 1.0)
+    S = DBTSystem(g, arc_angles(n, 7.5) if n > 1 else [0.0], device=dev)
+    p = torch.randn((n, nbx, nby), device=dev).to(dtype)
+    assert torch.equal(S.to_rows(p), p.transpose(1, 2))
