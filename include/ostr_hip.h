@@ -316,6 +316,10 @@ int ostr_prior_sart(ostr_handle* h, float* prior, const float* img, float delta,
  * (the taps' spectrum and the twiddles). */
 int ostr_fbp_filter(ostr_handle* h, float* q, const float* p, const float* taps, int32_t ntaps,
                     int32_t a0, int32_t a1, void* stream);
+/* ostr_fbp_filter with q detector-row-major [slot][nby][nbx], the layout
+ * ostr_bproj_sbp_rows takes (the same values). */
+int ostr_fbp_filter_rows(ostr_handle* h, float* q_rows, const float* p, const float* taps,
+                         int32_t ntaps, int32_t a0, int32_t a1, void* stream);
 
 /* ---- ReconDBT SART and ML (ReconDBT/SART_dbt.m, ML_dbt.m) on this build's
  * projector pair: G = ostr_fproj without cos, G^T = ostr_bproj_matched without

@@ -523,27 +523,41 @@ OSTR_API int ostr_line_integrals(ostr_handle* h, float* p, const float* y, const
     return e == hipSuccess ? OSTR_OK : hip_fail(h, e, "ostr_line_integrals");
 }
 
-OSTR_API int ostr_fbp_filter(ostr_handle* h, float* q, const float* p, const float* taps,
-                             int32_t ntaps, int32_t a0, int32_t a1, void* stream) {
-    CHECK_HANDLE(h);
+namespace {
+int fbp_filter(ostr_handle* h, float* q, const float* p, const float* taps, int32_t ntaps,
+               int32_t a0, int32_t a1, int rows, void* stream, const char* fn) {
     int rc;
-    if ((rc = check_range(h, a0, a1, "ostr_fbp_filter"))) return rc;
-    if (!q || !p || !taps || q == p) return fail(h, OSTR_E_ARG, "ostr_fbp_filter: bad buffers");
+    if ((rc = check_range(h, a0, a1, fn))) return rc;
+    if (!q || !p || !taps || q == p) return fail(h, OSTR_E_ARG, "%s: bad buffers", fn);
     if (ntaps <= 0 || ntaps % 2 == 0)
-        return fail(h, OSTR_E_ARG, "ostr_fbp_filter: ntaps must be odd and positive");
+        return fail(h, OSTR_E_ARG, "%s: ntaps must be odd and positive", fn);
     const int64_t L = (int64_t)1 << ostr::fbp_fft_log2(h->geom.nbx);
     if ((int64_t)(L + L / 2) * 8 > h->lds_limit)
         return fail(h, OSTR_E_RANGE,
-                    "ostr_fbp_filter: nbx=%d needs a %lld-point FFT, beyond the %d bytes of LDS "
+                    "%s: nbx=%d needs a %lld-point FFT, beyond the %d bytes of LDS "
                     "per work-group",
-                    h->geom.nbx, (long long)L, h->lds_limit);
+                    fn, h->geom.nbx, (long long)L, h->lds_limit);
     if ((rc = use_device(h))) return rc;
     hipStream_t st = (hipStream_t)stream;
-    if ((rc = ensure_work(h, (size_t)(L + L / 2) * sizeof(float2), st, "ostr_fbp_filter")))
+    if ((rc = ensure_work(h, (size_t)(L + L / 2) * sizeof(float2), st, fn)))
         return rc;
     hipError_t e = ostr::launch_fbp_filter(h->dg, h->views_dev, a0, a1, taps, ntaps, p,
-                                           (float2*)h->work, q, h->lds_limit, st);
-    return e == hipSuccess ? OSTR_OK : hip_fail(h, e, "ostr_fbp_filter (spectrum, FFT filter)");
+                                           (float2*)h->work, q, rows, h->lds_limit, st);
+    return e == hipSuccess ? OSTR_OK : hip_fail(h, e, fn);
+}
+}  // namespace
+
+OSTR_API int ostr_fbp_filter(ostr_handle* h, float* q, const float* p, const float* taps,
+                             int32_t ntaps, int32_t a0, int32_t a1, void* stream) {
+    CHECK_HANDLE(h);
+    return fbp_filter(h, q, p, taps, ntaps, a0, a1, 0, stream, "ostr_fbp_filter");
+}
+
+OSTR_API int ostr_fbp_filter_rows(ostr_handle* h, float* q_rows, const float* p,
+                                  const float* taps, int32_t ntaps, int32_t a0, int32_t a1,
+                                  void* stream) {
+    CHECK_HANDLE(h);
+    return fbp_filter(h, q_rows, p, taps, ntaps, a0, a1, 1, stream, "ostr_fbp_filter_rows");
 }
 
 // ---- ReconDBT SART / ML steps ------------------------------------------------

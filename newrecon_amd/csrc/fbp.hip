@@ -177,13 +177,14 @@ __device__ __forceinline__ int xcd_contiguous(int b, int n) {
 }
 
 // Group = SEQ column pairs (2 SEQ columns from j0) of one slot. LDS: L/2 + SEQ L
-// float2. p and q are [slot][nbx][nby] from slot a0; vec: nby % 4 == 0 and p,
-// q 16-byte aligned (SEQ = 2: float4 row loads and stores).
+// float2. p is [slot][nbx][nby] from slot a0, q the same or, with rows,
+// detector-row-major [slot][nby][nbx]; vec: nby % 4 == 0 and p, q 16-byte
+// aligned (SEQ = 2: float4 row loads and stores).
 template <int SEQ>
 __global__ __launch_bounds__(FFT_THREADS) void fbp_filter_kernel(
     DevGeom g, const ViewTab* __restrict__ views, int a0, int n_slots, int n_chunks, int logl,
     const float2* __restrict__ tw_g, const float2* __restrict__ hs, const float* __restrict__ p,
-    float* __restrict__ q, int vec) {
+    float* __restrict__ q, int vec, int rows) {
     extern __shared__ float2 lds[];
     const int L = 1 << logl;
     float2* tw = lds;
@@ -236,6 +237,19 @@ __global__ __launch_bounds__(FFT_THREADS) void fbp_filter_kernel(
         for (int s = 0; s < SEQ; ++s) buf[s * L + f] = cmul(buf[s * L + f], h);
     }
     fft_dif_inverse(buf, SEQ, logl, tw);
+    if (rows) {  // a detector row is contiguous: whole lines
+        const int64_t row0 = ((int64_t)slot * nby + j0) * nbx;
+        for (int i = threadIdx.x; i < nbx; i += FFT_THREADS) {
+            const unsigned r = bitrev((unsigned)i, logl);
+#pragma unroll
+            for (int s = 0; s < SEQ; ++s) {
+                const float2 y = buf[s * L + r];
+                if (j0 + 2 * s < nby) q[row0 + (int64_t)(2 * s) * nbx + i] = y.x;
+                if (j0 + 2 * s + 1 < nby) q[row0 + (int64_t)(2 * s + 1) * nbx + i] = y.y;
+            }
+        }
+        return;
+    }
     for (int i = threadIdx.x; i < nbx; i += FFT_THREADS) {
         const unsigned r = bitrev((unsigned)i, logl);
         float val[2 * SEQ];
@@ -272,7 +286,7 @@ int fbp_fft_log2(int nbx) {
 
 hipError_t launch_fbp_filter(const DevGeom& g, const ViewTab* views, int a0, int a1,
                              const float* taps, int ntaps, const float* p, float2* spec,
-                             float* q, int lds_limit, hipStream_t st) {
+                             float* q, int rows, int lds_limit, hipStream_t st) {
     const int n_slots = a1 - a0;
     if (n_slots <= 0) return hipSuccess;
     const int logl = fbp_fft_log2(g.nbx);
@@ -295,13 +309,13 @@ hipError_t launch_fbp_filter(const DevGeom& g, const ViewTab* views, int a0, int
         const int n_chunks = (g.nby + 3) / 4;
         hipLaunchKernelGGL(fbp_filter_kernel<2>, dim3((unsigned)(n_chunks * n_slots)),
                            dim3(FFT_THREADS), lds2, st, g, views, a0, n_slots, n_chunks, logl,
-                           tw, hs, p, q, vec);
+                           tw, hs, p, q, vec, rows);
     } else {
         if ((e = allow_lds((const void*)fbp_filter_kernel<1>, lds1)) != hipSuccess) return e;
         const int n_chunks = (g.nby + 1) / 2;
         hipLaunchKernelGGL(fbp_filter_kernel<1>, dim3((unsigned)(n_chunks * n_slots)),
                            dim3(FFT_THREADS), lds1, st, g, views, a0, n_slots, n_chunks, logl,
-                           tw, hs, p, q, 0);
+                           tw, hs, p, q, 0, rows);
     }
     return hipGetLastError();
 }

@@ -423,11 +423,12 @@ hipError_t launch_fill_f64(double* p, double v, int64_t n, hipStream_t st);
 // convolution along detector x with the centred taps, by FFT in LDS over
 // L = 2^fbp_fft_log2(nbx) >= 2 nbx - 1 points. spec: 3 L / 2 float2 of scratch
 // (twiddles and the taps' spectrum); lds_limit: the device's LDS bytes per
-// group (hipErrorInvalidValue when one column pair does not fit).
+// group (hipErrorInvalidValue when one column pair does not fit). rows: q
+// detector-row-major.
 int fbp_fft_log2(int nbx);
 hipError_t launch_fbp_filter(const DevGeom& g, const ViewTab* views, int a0, int a1,
                              const float* taps, int ntaps, const float* p, float2* spec,
-                             float* q, int lds_limit, hipStream_t st);
+                             float* q, int rows, int lds_limit, hipStream_t st);
 hipError_t launch_line_integrals(float* p, const float* y, const float* b, int64_t n,
                                  hipStream_t st);
 // Fused OSTR subset update with the exact transpose (hsub detector-row-major;

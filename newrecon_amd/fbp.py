@@ -65,5 +65,7 @@ def fbp_dbt(geom: Geometry, angles, proj, window: str = "hann", device=None):
     scale = math.pi / (nv * geom.dz)
     taps = torch.from_numpy((filter_taps(geom.nbx, geom.dbx, window) * scale)
                             .astype(np.float32)).to(dev)
-    q = S.fbp_filter(p, taps, 0, nv)
-    return S.bproj_sbp(q, 0, nv)
+    # filtered straight into the layout the backprojection gathers from: no
+    # transpose, and no work buffer of the sinogram's size
+    q = S.fbp_filter(p, taps, 0, nv, rows=True)
+    return S.bproj_sbp_rows(q, 0, nv)

@@ -98,6 +98,7 @@ def lib():
         "ostr_fproj_4r": [vp, vp, vp, vp, i32, i32, vp],
         "ostr_line_integrals": [vp, vp, vp, vp, i64, vp],
         "ostr_fbp_filter": [vp, vp, vp, vp, i32, i32, i32, vp],
+        "ostr_fbp_filter_rows": [vp, vp, vp, vp, i32, i32, i32, vp],
         "ostr_momentum_init": [vp, vp, vp],
         "ostr_update_fused_matched": [vp, vp, vp, i32, vp, vp, i32, i32, i32, f32, f32, i32, f32,
                                       f32, i32, vp],
@@ -513,15 +514,18 @@ class DBTSystem:
         """Tomo_OSTR.cu:2398: d_prjbuf [S][nby][nbx] = merged 2x2 sub-bin sums."""
         return self.fproj_4r(d_objbuf, angleStart, angleEnd, d_prjbuf, d_4R_prjbuf)
 
-    def fbp_filter(self, p, taps, a0, a1, q=None):
-        """Cosine-weighted views filtered along detector x with odd-length taps."""
-        q = self.sinogram(a1 - a0) if q is None else q
+    def fbp_filter(self, p, taps, a0, a1, q=None, rows=False):
+        """Cosine-weighted views filtered along detector x with odd-length taps;
+        rows: q detector-row-major [S][nby][nbx]."""
+        if q is None:
+            q = torch.empty((a1 - a0, self.geom.nby, self.geom.nbx), device=self.device) \
+                if rows else self.sinogram(a1 - a0)
         for t, what in ((p, "p"), (taps, "taps"), (q, "q")):
             _f32(t, what)
         if taps.numel() % 2 == 0:
             raise ValueError("FBP filter taps must have odd length")
-        self._check(self._L.ostr_fbp_filter(self._h, _p(q), _p(p), _p(taps), taps.numel(), a0,
-                                            a1, self._stream()))
+        fn = self._L.ostr_fbp_filter_rows if rows else self._L.ostr_fbp_filter
+        self._check(fn(self._h, _p(q), _p(p), _p(taps), taps.numel(), a0, a1, self._stream()))
         return q
 
     def line_integrals(self, y, b, p=None):
