@@ -11,17 +11,22 @@
 // q = IFFT(FFT(pw column) FFT(H)). Two real columns ride in one complex
 // sequence (column j real, j + 1 imaginary): H is real, so the convolution
 // keeps them apart. Per column pair a forward and an inverse radix-2 FFT
-// (L/2 log2 L butterflies each, two stages per LDS pass) replace the 2 nbx^2
-// multiply-adds of the direct sum.
+// (L/2 log2 L butterflies each) replace the 2 nbx^2 multiply-adds of the
+// direct sum.
 //
 // fbp_spectrum_kernel (one group) forms FFT(H) / L and the twiddle table
-// exp(-2 pi i k / L), k < L/2, rounded from double; fbp_filter_kernel gives
-// each group SEQ column pairs of one view: it loads them weighted and in
-// bit-reversed order into LDS, runs the decimation-in-time forward transform
-// (natural order out), multiplies by the spectrum, runs the
-// decimation-in-frequency inverse with conjugate twiddles (bit-reversed order
-// out) and stores rows i < nbx from their bit-reversed positions, so no
-// reordering pass is needed.
+// exp(-2 pi i k / L), k < L/2, rounded from double; the filter kernels give
+// each group SEQ column pairs of one view: they take them weighted and in
+// bit-reversed order, run the decimation-in-time forward transform (natural
+// order out), multiply by the spectrum, run the decimation-in-frequency
+// inverse with conjugate twiddles (bit-reversed order out) and store rows
+// i < nbx from their bit-reversed positions, so no reordering pass is needed.
+// From L = 1024 on fbp_filter_reg_kernel holds 16 points per thread and
+// sequence in registers through up to four radix-2 stages between LDS
+// exchanges; below that fbp_filter_kernel passes over LDS two stages at a time.
+// Both make the same operations.
+#include <type_traits>
+
 #include "ostr_internal.h"
 
 namespace ostr {
@@ -139,6 +144,126 @@ __device__ void fft_dif_inverse(float2* buf, int seq, int logl, const float2* tw
     __syncthreads();
 }
 
+// ---- 16 points per thread in registers --------------------------------------
+// L = 2^LOGL points, T = L / 16 threads. Pass p covers the radix-2 stages
+// 4p .. 4p + S - 1, S = min(4, LOGL - 4p): a thread holds 16 >> S whole groups of
+// 2^S points whose positions differ in those S bits only, so its stages need no
+// exchange. Between passes the points go through LDS; a thread writes where it
+// read in the pass before, so one barrier per exchange suffices. Positions are
+// swizzled (fft_swz) so that the 32 lanes of an 8-byte LDS access fall on
+// different banks in every pass (plain positions of pass 0 lie 128 bytes apart,
+// 16 lanes to a bank).
+template <int LOGL>
+struct FftPlan {
+    static constexpr int T = 1 << (LOGL - 4), PASSES = (LOGL + 3) / 4;
+    static constexpr int stages(int p) { return LOGL - 4 * p < 4 ? LOGL - 4 * p : 4; }
+};
+__device__ __forceinline__ int fft_swz(int i) { return i ^ ((i >> 4) & 31); }
+
+// Position of point q of group gg of thread t in pass P.
+template <int LOGL, int P>
+__device__ __forceinline__ int fft_pos(int t, int gg, int q) {
+    constexpr int S = FftPlan<LOGL>::stages(P), LG = 4 * P;
+    const int g = t + FftPlan<LOGL>::T * gg;
+    return ((g >> LG) << (LG + S)) | (q << LG) | (g & ((1 << LG) - 1));
+}
+
+// b times a twiddle (w or, conjugated, its mirror): index j of stage s of a group
+// at k = 0 is exp(-pi i j / 2^s), 1 for j = 0 and -i for j = 2^(s-1), for which
+// nothing is multiplied (the table holds these exactly, so the bits are the
+// same).
+template <bool INVERSE>
+__device__ __forceinline__ float2 fft_twiddle(float2 b, float2 w, int s, int j, bool at0) {
+    if (at0 && j == 0) return b;
+    if (at0 && 2 * j == (1 << s))
+        return INVERSE ? make_float2(-b.y, b.x) : make_float2(b.y, -b.x);
+    return cmul(b, w);
+}
+
+// Stages of pass P on the thread's points of SEQ sequences, e[seq][gg 2^S + q];
+// the twiddles are read once for all sequences. In pass 0 the group's k is 0.
+template <int LOGL, int SEQ, int P, bool INVERSE>
+__device__ __forceinline__ void fft_pass(float2 (&e)[SEQ][16], int t, const float2* tw) {
+    constexpr int S = FftPlan<LOGL>::stages(P), LG = 4 * P, N = 1 << S;
+#pragma unroll
+    for (int gg = 0; gg < 16 / N; ++gg) {
+        const int k = (t + FftPlan<LOGL>::T * gg) & ((1 << LG) - 1);
+        float2 w[N];  // stage s, index j at (1 << s) + j
+#pragma unroll
+        for (int s = 0; s < S; ++s)
+#pragma unroll
+            for (int j = 0; j < (1 << s); ++j) {
+                const float2 v = tw[(k + (j << LG)) << (LOGL - 1 - LG - s)];
+                w[(1 << s) + j] = INVERSE ? make_float2(v.x, -v.y) : v;
+            }
+#pragma unroll
+        for (int c = 0; c < SEQ; ++c) {
+            float2* a = e[c] + gg * N;
+#pragma unroll
+            for (int u = 0; u < S; ++u) {
+                const int s = INVERSE ? S - 1 - u : u;
+#pragma unroll
+                for (int q = 0; q < N; ++q) {
+                    if (q & (1 << s)) continue;
+                    const int j = q & ((1 << s) - 1);
+                    float2 &x = a[q], &y = a[q + (1 << s)];
+                    const float2 ws = w[(1 << s) + j];
+                    if (INVERSE) {
+                        const float2 d = csub(x, y);
+                        x = cadd(x, y);
+                        y = fft_twiddle<true>(d, ws, s, j, P == 0);
+                    } else {
+                        const float2 o = fft_twiddle<false>(y, ws, s, j, P == 0);
+                        y = csub(x, o);
+                        x = cadd(x, o);
+                    }
+                }
+            }
+        }
+    }
+}
+
+// The points from pass P's positions to pass Q's, through buf (SEQ L float2).
+template <int LOGL, int SEQ, int P, int Q>
+__device__ __forceinline__ void fft_exchange(float2 (&e)[SEQ][16], int t, float2* buf) {
+    constexpr int L = 1 << LOGL;
+    constexpr int NP = 1 << FftPlan<LOGL>::stages(P), NQ = 1 << FftPlan<LOGL>::stages(Q);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        const int at = fft_swz(fft_pos<LOGL, P>(t, i / NP, i % NP));
+#pragma unroll
+        for (int c = 0; c < SEQ; ++c) buf[c * L + at] = e[c][i];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        const int at = fft_swz(fft_pos<LOGL, Q>(t, i / NQ, i % NQ));
+#pragma unroll
+        for (int c = 0; c < SEQ; ++c) e[c][i] = buf[c * L + at];
+    }
+}
+
+// Forward transform from pass 0's positions (bit-reversed order in) to the last
+// pass' positions (natural order out); the inverse goes back the same way.
+template <int LOGL, int SEQ, int P = 0>
+__device__ __forceinline__ void fft_forward(float2 (&e)[SEQ][16], int t, float2* buf,
+                                            const float2* tw) {
+    fft_pass<LOGL, SEQ, P, false>(e, t, tw);
+    if constexpr (P + 1 < FftPlan<LOGL>::PASSES) {
+        fft_exchange<LOGL, SEQ, P, P + 1>(e, t, buf);
+        fft_forward<LOGL, SEQ, P + 1>(e, t, buf, tw);
+    }
+}
+template <int LOGL, int SEQ, int P = FftPlan<LOGL>::PASSES - 1>
+__device__ __forceinline__ void fft_inverse(float2 (&e)[SEQ][16], int t, float2* buf,
+                                            const float2* tw) {
+    fft_pass<LOGL, SEQ, P, true>(e, t, tw);
+    if constexpr (P > 0) {
+        fft_exchange<LOGL, SEQ, P, P - 1>(e, t, buf);
+        fft_inverse<LOGL, SEQ, P - 1>(e, t, buf, tw);
+    }
+}
+
 // One group: the twiddles tw (global, L/2) and hs = FFT(H) / L (global, L).
 // LDS: L + L/2 float2.
 __global__ __launch_bounds__(FFT_THREADS) void fbp_spectrum_kernel(const float* __restrict__ taps,
@@ -166,6 +291,47 @@ __global__ __launch_bounds__(FFT_THREADS) void fbp_spectrum_kernel(const float* 
     const float inv = 1.0f / (float)L;  // a power of two: exact
     for (int p = threadIdx.x; p < L; p += FFT_THREADS)
         hs[p] = make_float2(a[p].x * inv, a[p].y * inv);
+}
+
+// fbp_spectrum_kernel with 16 points per thread in registers (L / 16 threads).
+// The twiddles come from the first octant, the rest by symmetry: in double,
+// one CU's share of 2048 sine and cosine pairs took longer than the transform.
+template <int LOGL>
+__global__ __launch_bounds__(FftPlan<LOGL>::T) void fbp_spectrum_reg_kernel(
+    const float* __restrict__ taps, int ntaps, int nbx, float2* __restrict__ tw_out,
+    float2* __restrict__ hs) {
+    extern __shared__ float2 lds[];
+    constexpr int L = 1 << LOGL, T = FftPlan<LOGL>::T, LAST = FftPlan<LOGL>::PASSES - 1;
+    float2* tw = lds;
+    float2* buf = lds + L / 2;
+    const int t = threadIdx.x, c = (ntaps - 1) / 2;
+    float2 e[1][16];
+#pragma unroll
+    for (int m = 0; m < 16; ++m) {
+        const int pos = (int)bitrev((unsigned)(16 * t + m), LOGL);
+        const int k = pos < L / 2 ? pos : pos - L;
+        const int i = c - k;
+        const bool on = k >= -(nbx - 1) && k <= nbx - 1 && i >= 0 && i < ntaps;
+        e[0][m] = make_float2(on ? taps[i] : 0.0f, 0.0f);
+    }
+    for (int k = t; k <= L / 8; k += T) {
+        double sn, cs;
+        sincospi(2.0 * (double)k / (double)L, &sn, &cs);
+        const float x = (float)cs, y = (float)sn;
+        tw[k] = make_float2(x, -y);
+        tw[L / 4 - k] = make_float2(y, -x);
+        tw[L / 4 + k] = make_float2(-y, -x);
+        if (k) tw[L / 2 - k] = make_float2(-x, -y);
+    }
+    __syncthreads();
+    for (int k = t; k < L / 2; k += T) tw_out[k] = tw[k];
+    fft_forward<LOGL, 1>(e, t, buf, tw);
+    const float inv = 1.0f / (float)L;  // a power of two: exact
+#pragma unroll
+    for (int m = 0; m < 16; ++m) {
+        constexpr int N = 1 << FftPlan<LOGL>::stages(LAST);
+        hs[fft_pos<LOGL, LAST>(t, m / N, m % N)] = make_float2(e[0][m].x * inv, e[0][m].y * inv);
+    }
 }
 
 // Group b of an n-group launch runs on XCD b % 8; hand each XCD one contiguous
@@ -270,6 +436,123 @@ __global__ __launch_bounds__(FFT_THREADS) void fbp_filter_kernel(
     }
 }
 
+// fbp_filter_kernel with 16 points per thread and sequence in registers: same
+// task and buffers, L / 16 threads. The forward transform's last pass, the
+// spectrum and the inverse's first pass work on the same points, so 4 LDS
+// exchanges at L = 4096 (one more for ROWS, detector-row-major q) replace 14
+// passes over LDS. Bound by VALU issue (two waves per SIMD, 245 VGPRs) and the
+// 16-byte pieces of p. 9 views of 2048x1664 bins:
+// 365 us in passes, 174 here (ROWS 179); 25 of 1106x777 460, 253 (ROWS 210).
+template <int LOGL, int SEQ, bool ROWS>
+__global__ __launch_bounds__(FftPlan<LOGL>::T) __attribute__((amdgpu_waves_per_eu(2)))
+void fbp_filter_reg_kernel(
+    DevGeom g, const ViewTab* __restrict__ views, int a0, int n_slots, int n_chunks,
+    const float2* __restrict__ tw_g, const float2* __restrict__ hs, const float* __restrict__ p,
+    float* __restrict__ q, int vec) {
+    extern __shared__ float2 lds[];
+    constexpr int L = 1 << LOGL, T = FftPlan<LOGL>::T, LAST = FftPlan<LOGL>::PASSES - 1;
+    float2* tw = lds;
+    float2* buf = lds + L / 2;
+    const int t = threadIdx.x;
+    const int task = xcd_contiguous((int)blockIdx.x, n_chunks * n_slots);
+    const int slot = task / n_chunks;
+    const int j0 = (task % n_chunks) * 2 * SEQ;
+    const int nbx = g.nbx, nby = g.nby;
+    const ViewTab v = views[a0 + slot];
+    const float D = v.z0 + g.det_r;
+    float dy[2 * SEQ];
+#pragma unroll
+    for (int c = 0; c < 2 * SEQ; ++c) {
+        const float ey = (float)((double)g.y_d0 + ((double)(j0 + c) + 0.5) * (double)g.dby);
+        dy[c] = ey - g.src_y;
+    }
+    const int64_t base = (int64_t)slot * nbx * nby + j0;
+    // the column pairs' rows in bit-reversed order, all loads first
+    float2 e[SEQ][16];
+#pragma unroll
+    for (int m = 0; m < 16; ++m) {
+        const int i = (int)bitrev((unsigned)(16 * t + m), LOGL);
+        float val[2 * SEQ];
+#pragma unroll
+        for (int c = 0; c < 2 * SEQ; ++c) val[c] = 0.0f;
+        if (i < nbx) {
+            const float* row = p + base + (int64_t)i * nby;
+            if (SEQ == 2 && vec) {
+                const float4 r4 = *(const float4*)row;
+                val[0] = r4.x;
+                val[1] = r4.y;
+                val[2 * SEQ - 2] = r4.z;
+                val[2 * SEQ - 1] = r4.w;
+            } else {
+#pragma unroll
+                for (int c = 0; c < 2 * SEQ; ++c) val[c] = j0 + c < nby ? row[c] : 0.0f;
+            }
+        }
+#pragma unroll
+        for (int c = 0; c < SEQ; ++c) e[c][m] = make_float2(val[2 * c], val[2 * c + 1]);
+    }
+    for (int k = t; k < L / 2; k += T) tw[k] = tw_g[k];
+#pragma unroll
+    for (int m = 0; m < 16; ++m) {
+        const int i = (int)bitrev((unsigned)(16 * t + m), LOGL);
+        if (i >= nbx) continue;
+        const float ex = (float)((double)g.x_d0 + ((double)i + 0.5) * (double)g.dbx);
+        const float dx = ex - v.x0;
+#pragma unroll
+        for (int c = 0; c < SEQ; ++c) {
+            e[c][m].x *= D / sqrtf(fmaf(dx, dx, fmaf(dy[2 * c], dy[2 * c], D * D)));
+            e[c][m].y *= D / sqrtf(fmaf(dx, dx, fmaf(dy[2 * c + 1], dy[2 * c + 1], D * D)));
+        }
+    }
+    __syncthreads();
+    fft_forward<LOGL, SEQ>(e, t, buf, tw);
+#pragma unroll
+    for (int m = 0; m < 16; ++m) {
+        constexpr int N = 1 << FftPlan<LOGL>::stages(LAST);
+        const float2 h = hs[fft_pos<LOGL, LAST>(t, m / N, m % N)];
+#pragma unroll
+        for (int c = 0; c < SEQ; ++c) e[c][m] = cmul(e[c][m], h);
+    }
+    fft_inverse<LOGL, SEQ>(e, t, buf, tw);
+    if (ROWS) {
+        // through LDS once more, so that a wave writes whole lines of a row;
+        // positions swizzled for the bit-reversed writes (8 lanes to a bank)
+        __syncthreads();
+        auto swz = [](int i) { return i ^ ((i >> 3) & 31); };
+#pragma unroll
+        for (int m = 0; m < 16; ++m) {
+            const int i = (int)bitrev((unsigned)(16 * t + m), LOGL);
+#pragma unroll
+            for (int c = 0; c < SEQ; ++c) buf[c * L + swz(i)] = e[c][m];
+        }
+        __syncthreads();
+        float* row = q + ((int64_t)slot * nby + j0) * nbx;
+        for (int i = t; i < nbx; i += T) {
+#pragma unroll
+            for (int c = 0; c < SEQ; ++c) {
+                const float2 y = buf[c * L + swz(i)];
+                if (j0 + 2 * c < nby) row[(int64_t)(2 * c) * nbx + i] = y.x;
+                if (j0 + 2 * c + 1 < nby) row[(int64_t)(2 * c + 1) * nbx + i] = y.y;
+            }
+        }
+        return;
+    }
+#pragma unroll
+    for (int m = 0; m < 16; ++m) {
+        const int i = (int)bitrev((unsigned)(16 * t + m), LOGL);
+        if (i >= nbx) continue;
+        float* row = q + base + (int64_t)i * nby;
+        if (SEQ == 2 && vec) {
+            *(float4*)row =
+                make_float4(e[0][m].x, e[0][m].y, e[SEQ - 1][m].x, e[SEQ - 1][m].y);
+        } else {
+#pragma unroll
+            for (int c = 0; c < 2 * SEQ; ++c)
+                if (j0 + c < nby) row[c] = (c & 1) ? e[c / 2][m].y : e[c / 2][m].x;
+        }
+    }
+}
+
 // Dynamic LDS beyond 64 KiB per group needs the kernel's opt-in.
 hipError_t allow_lds(const void* kernel, size_t bytes) {
     if (bytes <= 65536) return hipSuccess;
@@ -297,26 +580,52 @@ hipError_t launch_fbp_filter(const DevGeom& g, const ViewTab* views, int a0, int
     const size_t lds2 = (size_t)(L / 2 + 2 * L) * sizeof(float2);
     const size_t lds1 = (size_t)(L / 2 + L) * sizeof(float2);
     if (lds1 > (size_t)lds_limit || spec_lds > (size_t)lds_limit) return hipErrorInvalidValue;
-    hipError_t e = allow_lds((const void*)fbp_spectrum_kernel, spec_lds);
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(fbp_spectrum_kernel, dim3(1), dim3(FFT_THREADS), spec_lds, st, taps,
-                       ntaps, g.nbx, logl, tw, hs);
-    e = hipGetLastError();
-    if (e != hipSuccess) return e;
     const int vec = (g.nby % 4 == 0) && ((uintptr_t)p % 16 == 0) && ((uintptr_t)q % 16 == 0);
-    if (lds2 <= (size_t)lds_limit) {
-        if ((e = allow_lds((const void*)fbp_filter_kernel<2>, lds2)) != hipSuccess) return e;
-        const int n_chunks = (g.nby + 3) / 4;
-        hipLaunchKernelGGL(fbp_filter_kernel<2>, dim3((unsigned)(n_chunks * n_slots)),
-                           dim3(FFT_THREADS), lds2, st, g, views, a0, n_slots, n_chunks, logl,
-                           tw, hs, p, q, vec, rows);
-    } else {
-        if ((e = allow_lds((const void*)fbp_filter_kernel<1>, lds1)) != hipSuccess) return e;
-        const int n_chunks = (g.nby + 1) / 2;
-        hipLaunchKernelGGL(fbp_filter_kernel<1>, dim3((unsigned)(n_chunks * n_slots)),
-                           dim3(FFT_THREADS), lds1, st, g, views, a0, n_slots, n_chunks, logl,
-                           tw, hs, p, q, 0, rows);
+    // two column pairs per group where they fit (at 8192 points in registers one)
+    const bool two = lds2 <= (size_t)lds_limit && logl < 13;
+    const int n_chunks = two ? (g.nby + 3) / 4 : (g.nby + 1) / 2;
+    const dim3 grid((unsigned)(n_chunks * n_slots));
+    const size_t lds = two ? lds2 : lds1;
+    // at most 1024 points; 256 threads, which one wave of 16 points each is slower than
+    auto spectrum_by_passes = [&] {
+        hipLaunchKernelGGL(fbp_spectrum_kernel, dim3(1), dim3(FFT_THREADS), spec_lds, st, taps,
+                           ntaps, g.nbx, logl, tw, hs);
+        return hipGetLastError();
+    };
+    auto in_registers = [&](auto logl_c, auto seq_c) {
+        constexpr int LOGL = decltype(logl_c)::value, SEQ = decltype(seq_c)::value;
+        const auto kernel = rows ? fbp_filter_reg_kernel<LOGL, SEQ, true>
+                                 : fbp_filter_reg_kernel<LOGL, SEQ, false>;
+        hipError_t err = allow_lds((const void*)kernel, lds);
+        if (err != hipSuccess) return err;
+        if constexpr (LOGL > 10) {
+            const auto spectrum = fbp_spectrum_reg_kernel<LOGL>;
+            if ((err = allow_lds((const void*)spectrum, spec_lds)) != hipSuccess) return err;
+            hipLaunchKernelGGL(spectrum, dim3(1), dim3(FftPlan<LOGL>::T), spec_lds, st, taps,
+                               ntaps, g.nbx, tw, hs);
+            if ((err = hipGetLastError()) != hipSuccess) return err;
+        } else if ((err = spectrum_by_passes()) != hipSuccess) {
+            return err;
+        }
+        hipLaunchKernelGGL(kernel, grid, dim3(FftPlan<LOGL>::T), lds, st, g, views, a0, n_slots,
+                           n_chunks, tw, hs, p, q, SEQ == 2 ? vec : 0);
+        return hipGetLastError();
+    };
+    auto by_seq = [&](auto logl_c) {
+        return two ? in_registers(logl_c, std::integral_constant<int, 2>())
+                   : in_registers(logl_c, std::integral_constant<int, 1>());
+    };
+    switch (logl) {
+        case 10: return by_seq(std::integral_constant<int, 10>());
+        case 11: return by_seq(std::integral_constant<int, 11>());
+        case 12: return by_seq(std::integral_constant<int, 12>());
+        case 13: return by_seq(std::integral_constant<int, 13>());
     }
+    // fewer than 64 threads of 16 points: passes over LDS
+    const hipError_t e = spectrum_by_passes();
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(fbp_filter_kernel<2>, grid, dim3(FFT_THREADS), lds, st, g, views, a0,
+                       n_slots, n_chunks, logl, tw, hs, p, q, vec, rows);
     return hipGetLastError();
 }
 
