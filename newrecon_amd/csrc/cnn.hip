@@ -45,6 +45,12 @@ constexpr int kpad(int cin) { return ((27 * cin + 31) / 32) * 32; }
 __device__ __forceinline__ u16 to_bf16(float v) { return bf16_bits(v); }
 __device__ __forceinline__ float from_bf16(u16 b) { return __uint_as_float((uint32_t)b << 16); }
 
+// two floats to BF16 (round to nearest even) in one conversion instruction
+__device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) {
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t, bf16x2{(__bf16)lo, (__bf16)hi});
+}
+
 __device__ __forceinline__ bf16x8 load8(const u16* p) {
     return *reinterpret_cast<const bf16x8*>(p);
 }
@@ -71,13 +77,31 @@ __device__ __forceinline__ bf16x8 zero8() {
 // (p / NC8) % 3, p % NC8) (pairs past 9 NC8 get zero weights), so the B
 // operand of input row r and chunk q serves output rows r - dyi, dyi = dy + 1,
 // of all three dy: (R + 2) LDS reads per 3 R MFMAs per column block and
-// output-channel block. A operands are read from the packed weights
-// (tap * CIN + 8 c8, 16 bytes): all of them once, into registers, where they
-// fit, else one chunk ahead.
+// output-channel block. A operands come from the packed weights
+// (tap * CIN + 8 c8, 16 bytes): read once into registers where they fit, else
+// once into LDS where they fit beside the slabs, else per chunk (a step's global
+// loads wait for the step before's stores, see the epilogue). At 256x256x48
+// voxels, weights per chunk and in LDS: 16->48 345 and 270 us, 16->32 33 and 27
+// (128x128x24), 32->32 72 and 42, 32->64 25 and 16 (64x64x12).
 // Slab elements per LDS slot, and loader waves: each holds at most 24 of its
 // 16-byte elements per lane in flight.
 constexpr int conv_slab(int cin, int r, int xw) { return cin / 8 * (4 * r + 2) * (xw + 2); }
 constexpr int conv_loaders(int slab) { return (slab + 64 * 24 - 1) / (64 * 24); }
+
+// Weights of a wave in registers (the rule and its budget are in the kernel),
+// else in LDS if they fit beside the slabs, else read per chunk.
+constexpr int conv_chunks(int cin) { return (9 * (cin / 8) + 3) / 4; }
+constexpr bool conv_weights_in_registers(int cin, int cout, int r, int xw) {
+    const bool pipe = r == 1 && cout == 16;
+    const int acc = 4 * r * (xw / 16) * (cout / 16) + (pipe ? 4 * (r + 2) * (xw / 16) : 0);
+    return 12 * conv_chunks(cin) * (cout / 16) + acc <= (pipe ? 220 : 180);
+}
+constexpr int conv_slab_bytes(int cin, int r, int xw) { return (3 * conv_slab(cin, r, xw) + 64) * 16; }
+constexpr int conv_weight_bytes(int cin, int cout) { return conv_chunks(cin) * 3 * (cout / 16) * 1024; }
+constexpr bool conv_weights_in_lds(int cin, int cout, int r, int xw) {
+    return !conv_weights_in_registers(cin, cout, r, xw) &&
+           conv_slab_bytes(cin, r, xw) + conv_weight_bytes(cin, cout) <= 160 * 1024;
+}
 
 template <int CIN, int COUT, int R, int XW>
 __global__ __launch_bounds__(256 + 64 * conv_loaders(conv_slab(CIN, R, XW))) void conv3d_lds_kernel(
@@ -89,7 +113,7 @@ __global__ __launch_bounds__(256 + 64 * conv_loaders(conv_slab(CIN, R, XW))) voi
     constexpr int KP = kpad(CIN), NCO = COUT / 16, NVB = XW / 16;
     constexpr int TR = 4 * R + 2, TW = XW + 2, SLAB = conv_slab(CIN, R, XW);
     constexpr int LW = conv_loaders(SLAB), NT = 256 + 64 * LW;
-    extern __shared__ uint4 slabs[];  // 3 * SLAB
+    extern __shared__ uint4 slabs[];  // 3 * SLAB, then one place per lane
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int n = lane & 15, kg = lane >> 4;
     // group b runs on XCD b % 8: give each XCD a contiguous range of tiles so
@@ -106,63 +130,27 @@ __global__ __launch_bounds__(256 + 64 * conv_loaders(conv_slab(CIN, R, XW))) voi
     const int x0 = tx * XW, y0 = ty * 4 * R, z0 = tz * zc;
     const int z1 = z0 + zc < nz ? z0 + zc : nz;
 
-    // slab element e -> (row, xi, c8), c8 fastest (contiguous global reads)
-    auto src_of = [&](int e, int zi, bool& ok) -> const uint4* {
+    // Slab element e -> (row, xi, c8), c8 fastest (contiguous global reads): its
+    // offset inside a slice of x, in 16-byte units, and its place in an LDS
+    // slot, both the same for every slice. Elements outside the volume's x, y
+    // range are zero in all slots from the start; their later loads read the
+    // slice's first element and go to a place of the lane's own past the slabs.
+    const int xs8 = xcs / 8;
+    const u16* xb = x + xco;
+    const int64_t slice = (int64_t)ny * nx * xcs;
+    auto place = [&](int e, uint32_t& off, int& at) -> bool {
         const int c8 = e % NC8, rest = e / NC8;
         const int xi = rest % TW, row = rest / TW;
         const int gx = x0 - 1 + xi, gy = y0 - 1 + row;
-        ok = e < SLAB && (unsigned)zi < (unsigned)nz && (unsigned)gx < (unsigned)nx &&
-             (unsigned)gy < (unsigned)ny;
-        return reinterpret_cast<const uint4*>(x + (((int64_t)zi * ny + gy) * nx + gx) * xcs +
-                                              xco + c8 * 8);
+        const bool ok = e < SLAB && (unsigned)gx < (unsigned)nx && (unsigned)gy < (unsigned)ny;
+        off = ok ? (uint32_t)(gy * nx + gx) * (uint32_t)xs8 + (uint32_t)c8 : 0u;
+        at = (c8 * TR + row) * TW + xi;
+        return ok;
     };
-    auto dst_of = [&](int e, int zi) -> uint4* {
-        const int c8 = e % NC8, rest = e / NC8;
-        const int xi = rest % TW, row = rest / TW;
-        return slabs + ((zi + 3) % 3) * SLAB + (c8 * TR + row) * TW + xi;
+    auto slot_of = [&](int zi) { return slabs + ((zi + 3) % 3) * SLAB; };
+    auto element = [&](int zi, uint32_t off) {
+        return reinterpret_cast<const uint4*>(xb + zi * slice) + off;
     };
-
-    // the first three slabs, by all waves
-    for (int zi = z0 - 1; zi <= z0 + 1; ++zi) {
-        constexpr int NA = (SLAB + NT - 1) / NT;
-        uint4 v[NA];
-#pragma unroll
-        for (int i = 0; i < NA; ++i) {
-            bool ok;
-            const uint4* src = src_of((int)threadIdx.x + NT * i, zi, ok);
-            v[i] = ok ? *src : make_uint4(0u, 0u, 0u, 0u);
-        }
-#pragma unroll
-        for (int i = 0; i < NA; ++i) {
-            const int e = (int)threadIdx.x + NT * i;
-            if (e < SLAB) *dst_of(e, zi) = v[i];
-        }
-    }
-    __syncthreads();
-
-    if (wave >= 4) {
-        // loaders: slab z + 2 in registers during step z, stored between the barriers
-        constexpr int NL = (SLAB + 64 * LW - 1) / (64 * LW);
-        const int l0 = (int)threadIdx.x - 256;
-#pragma unroll 1
-        for (int z = z0; z + 1 < z1; ++z) {
-            uint4 v[NL];
-#pragma unroll
-            for (int i = 0; i < NL; ++i) {
-                bool ok;
-                const uint4* src = src_of(l0 + 64 * LW * i, z + 2, ok);
-                v[i] = ok ? *src : make_uint4(0u, 0u, 0u, 0u);
-            }
-            __syncthreads();  // slice z - 1's slot is read no more
-#pragma unroll
-            for (int i = 0; i < NL; ++i) {
-                const int e = l0 + 64 * LW * i;
-                if (e < SLAB) *dst_of(e, z + 2) = v[i];
-            }
-            __syncthreads();
-        }
-        return;
-    }
 
     auto load_a = [&](int q, bf16x8 (&a)[3][NCO]) {
         const int p = 4 * q + kg;
@@ -175,6 +163,91 @@ __global__ __launch_bounds__(256 + 64 * conv_loaders(conv_slab(CIN, R, XW))) voi
                                             (dzi * 9 + dyi * 3 + dxi) * CIN + c8 * 8)
                                     : zero8();
     };
+    // Weights in LDS as the operands' register image, [q][dyi][cb][lane], each
+    // read 1 KB of consecutive 16-byte elements; written by all waves, read
+    // after the barrier below.
+    constexpr bool WLDS = conv_weights_in_lds(CIN, COUT, R, XW);
+    bf16x8* wl = reinterpret_cast<bf16x8*>(slabs + 3 * SLAB + 64);
+    if constexpr (WLDS) {
+#pragma unroll 1
+        for (int q = wave; q < NQ; q += NT / 64) {
+            bf16x8 a[3][NCO];
+            load_a(q, a);
+#pragma unroll
+            for (int d = 0; d < 3; ++d)
+#pragma unroll
+                for (int cb = 0; cb < NCO; ++cb) wl[((q * 3 + d) * NCO + cb) * 64 + lane] = a[d][cb];
+        }
+    }
+
+    // the first three slabs, by all waves
+    {
+        constexpr int NA = (SLAB + NT - 1) / NT;
+        for (int zi = z0 - 1; zi <= z0 + 1; ++zi) {
+            const bool in = (unsigned)zi < (unsigned)nz;
+            uint4* dst = slot_of(zi);
+            uint4 v[NA];
+#pragma unroll
+            for (int i = 0; i < NA; ++i) {
+                uint32_t off;
+                int at;
+                const bool ok = place((int)threadIdx.x + NT * i, off, at);
+                v[i] = make_uint4(0u, 0u, 0u, 0u);
+                if (ok && in) v[i] = *element(zi, off);
+            }
+#pragma unroll
+            for (int i = 0; i < NA; ++i) {
+                const int e = (int)threadIdx.x + NT * i;
+                uint32_t off;
+                int at;
+                place(e, off, at);
+                if (e < SLAB) dst[at] = v[i];
+            }
+        }
+    }
+    __syncthreads();
+
+    if (wave >= 4) {
+        // Loaders: slab z + 2 in registers during step z, stored between the
+        // barriers. Nothing but a load and a store per element is left to do in
+        // a step: with the offsets and range checks formed per element and
+        // slice the loader's ~1000 instructions set the pace of the group.
+        constexpr int NL = (SLAB + 64 * LW - 1) / (64 * LW);
+        const int l0 = (int)threadIdx.x - 256;
+        uint32_t off[NL];
+        int at[NL];
+#pragma unroll
+        for (int i = 0; i < NL; ++i)
+            if (!place(l0 + 64 * LW * i, off[i], at[i])) at[i] = -1;
+#pragma unroll 1
+        for (int z = z0; z + 1 < z1; ++z) {
+            uint4 v[NL];
+            if (z + 2 < nz) {
+#pragma unroll
+                for (int i = 0; i < NL; ++i) v[i] = *element(z + 2, off[i]);
+            } else {
+#pragma unroll
+                for (int i = 0; i < NL; ++i) v[i] = make_uint4(0u, 0u, 0u, 0u);
+            }
+            __syncthreads();  // slice z - 1's slot is read no more
+            const int s0 = ((z + 2) % 3) * SLAB;
+#pragma unroll
+            for (int i = 0; i < NL; ++i) slabs[at[i] < 0 ? 3 * SLAB + lane : s0 + at[i]] = v[i];
+            __syncthreads();
+        }
+        return;
+    }
+
+    auto operands = [&](int q, bf16x8 (&a)[3][NCO]) {
+        if constexpr (WLDS) {
+#pragma unroll
+            for (int d = 0; d < 3; ++d)
+#pragma unroll
+                for (int cb = 0; cb < NCO; ++cb) a[d][cb] = wl[((q * 3 + d) * NCO + cb) * 64 + lane];
+        } else {
+            load_a(q, a);
+        }
+    };
     // B operands: row r of chunk q is read from LDS two row steps before its
     // MFMAs, into slot r of a ring of R + 2 row buffers (the reads of the next
     // chunk's rows 0 and 1 overlap this chunk's last two rows); scheduling
@@ -185,7 +258,9 @@ __global__ __launch_bounds__(256 + 64 * conv_loaders(conv_slab(CIN, R, XW))) voi
         // pairs past the last read a valid slab element (their weights are 0)
         const int p = 4 * q + kg < NP ? 4 * q + kg : NP - 1;
         const int c8 = p % NC8, dxi = (p / NC8) % 3, dzi = p / (3 * NC8);
-        return slabs + ((z + dzi + 2) % 3) * SLAB + (c8 * TR + wave * R) * TW + n + dxi;
+        const int m = (z + 2) % 3;  // slot of slice z - 1
+        const int s0 = m * SLAB, s1 = (m == 2 ? 0 : m + 1) * SLAB, s2 = (m == 0 ? 2 : m - 1) * SLAB;
+        return slabs + (dzi == 0 ? s0 : dzi == 1 ? s1 : s2) + (c8 * TR + wave * R) * TW + n + dxi;
     };
     bf16x8 ring[PIPE ? RR : 1][NVB];
     auto read_row = [&](const uint4* bp, int r, bf16x8 (&dst)[NVB]) {
@@ -253,20 +328,53 @@ __global__ __launch_bounds__(256 + 64 * conv_loaders(conv_slab(CIN, R, XW))) voi
     // VGPR budget (256 per lane: a group of 5-6 waves puts two on some SIMD).
     // The weights stay in registers for the whole kernel when they, the
     // accumulators and the row ring fit (in 220 VGPRs; 180 where the compiler
-    // schedules the reads); otherwise each chunk's are loaded one chunk ahead,
-    // or at the chunk where two chunks' would not fit.
+    // schedules the reads: conv_weights_in_registers); otherwise each chunk's
+    // are read one chunk ahead, or at the chunk where two chunks' would not fit.
     constexpr int ACC = 4 * R * NVB * NCO + (PIPE ? 4 * RR * NVB : 0);
-    constexpr bool AREG = 12 * NQ * NCO + ACC <= (PIPE ? 220 : 180);
+    constexpr bool AREG = conv_weights_in_registers(CIN, COUT, R, XW);
     constexpr int NQR = AREG ? NQ : 1, NQA = AREG || 24 * NCO + ACC > 200 ? 1 : 2;
     bf16x8 aw[NQR][3][NCO], ab[NQA][3][NCO];
     if constexpr (AREG) {
 #pragma unroll
         for (int q = 0; q < NQ; ++q) load_a(q, aw[q]);
     } else if constexpr (NQA == 2) {
-        load_a(0, ab[0]);
+        operands(0, ab[0]);
     }
+    // A wave's memory counter is in order and counts stores: a load asked for
+    // in the epilogue would wait for the step before's stores to reach memory.
+    // So the bias is loaded once, the weights come from registers or LDS where
+    // they fit, and the ReLU masks of a step (4 channels = 8 bytes per output)
+    // are loaded before its MFMAs where registers allow. With all three in the
+    // step, 16->16 channels at 256x256x48 voxels took 127 us, now 92.
+    constexpr bool MASKS_FIRST = 2 * R * NVB * NCO <= 16;
+    float4 bv[NCO];
+#pragma unroll
+    for (int cb = 0; cb < NCO; ++cb)
+        bv[cb] = bias ? *reinterpret_cast<const float4*>(bias + cb * 16 + kg * 4)
+                      : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
 #pragma unroll 1
     for (int z = z0; z < z1; ++z) {
+        // voxel (x0 + n, first row) of this lane; the others lie a wave-uniform
+        // number of voxels on
+        const int gx0 = x0 + n, gy0 = y0 + wave * R;
+        const int64_t v0 = ((int64_t)z * ny + gy0) * nx + gx0;
+        u16* yp = y + v0 * ycs + yco + kg * 4;
+        const u16* mp = mask + v0 * mcs + mco + kg * 4;
+        uint2 mk[R][NVB][NCO];
+        auto load_masks = [&] {
+#pragma unroll
+            for (int o = 0; o < R; ++o)
+#pragma unroll
+                for (int nb = 0; nb < NVB; ++nb)
+#pragma unroll
+                    for (int cb = 0; cb < NCO; ++cb) {
+                        mk[o][nb][cb] = make_uint2(0xFFFFFFFFu, 0xFFFFFFFFu);
+                        if (mask && gy0 + o < ny && gx0 + nb * 16 < nx)
+                            mk[o][nb][cb] = *reinterpret_cast<const uint2*>(
+                                mp + (int64_t)(o * nx + nb * 16) * mcs + cb * 16);
+                    }
+        };
+        if constexpr (MASKS_FIRST) load_masks();
         f32x4 acc[R][NVB][NCO];
 #pragma unroll
         for (int o = 0; o < R; ++o)
@@ -287,66 +395,44 @@ __global__ __launch_bounds__(256 + 64 * conv_loaders(conv_slab(CIN, R, XW))) voi
             for (int q = 0; q < NQ; ++q) {
                 if constexpr (NQA == 2) {
                     // after the last chunk: the next slice's first
-                    load_a(q + 1 < NQ ? q + 1 : 0, ab[NQA - 1]);
+                    operands(q + 1 < NQ ? q + 1 : 0, ab[NQA - 1]);
                     chunk(z, q, bq, ab[0], acc);
 #pragma unroll
                     for (int dyi = 0; dyi < 3; ++dyi)
 #pragma unroll
                         for (int cb = 0; cb < NCO; ++cb) ab[0][dyi][cb] = ab[NQA - 1][dyi][cb];
                 } else {
-                    load_a(q, ab[0]);
+                    operands(q, ab[0]);
                     chunk(z, q, bq, ab[0], acc);
                 }
             }
         }
-        // epilogue: the bias and the ReLU masks of all outputs first (4 channels
-        // = 8 bytes), then the stores
-        float4 bv[NCO];
-#pragma unroll
-        for (int cb = 0; cb < NCO; ++cb)
-            bv[cb] = bias ? *reinterpret_cast<const float4*>(bias + cb * 16 + kg * 4)
-                          : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        uint2 mk[R][NVB][NCO];
-#pragma unroll
-        for (int o = 0; o < R; ++o)
-#pragma unroll
-            for (int nb = 0; nb < NVB; ++nb)
-#pragma unroll
-                for (int cb = 0; cb < NCO; ++cb) {
-                    const int gy = y0 + wave * R + o, gx = x0 + nb * 16 + n;
-                    const int64_t v = ((int64_t)z * ny + gy) * nx + gx;
-                    mk[o][nb][cb] = make_uint2(0xFFFFFFFFu, 0xFFFFFFFFu);
-                    if (mask && gy < ny && gx < nx)
-                        mk[o][nb][cb] = *reinterpret_cast<const uint2*>(
-                            mask + v * mcs + mco + cb * 16 + kg * 4);
-                }
+        // epilogue
+        if constexpr (!MASKS_FIRST) load_masks();
 #pragma unroll
         for (int o = 0; o < R; ++o) {
-            const int gy = y0 + wave * R + o;
-            if (gy >= ny) continue;
+            if (gy0 + o >= ny) continue;
 #pragma unroll
             for (int nb = 0; nb < NVB; ++nb) {
-                const int gx = x0 + nb * 16 + n;
-                if (gx >= nx) continue;
-                const int64_t v = ((int64_t)z * ny + gy) * nx + gx;
+                if (gx0 + nb * 16 >= nx) continue;
+                u16* yv = yp + (int64_t)(o * nx + nb * 16) * ycs;
 #pragma unroll
                 for (int cb = 0; cb < NCO; ++cb) {
-                    const int c0 = cb * 16 + kg * 4;
                     const uint32_t m2[2] = {mk[o][nb][cb].x, mk[o][nb][cb].y};
-                    u16 ov[4];
+                    float val[4];
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
-                        float val = acc[o][nb][cb][e];
-                        if (bias) val += e == 0 ? bv[cb].x : e == 1 ? bv[cb].y : e == 2 ? bv[cb].z : bv[cb].w;
-                        if (relu) val = val > 0.0f ? val : 0.0f;
+                        val[e] = acc[o][nb][cb][e];
+                        if (bias)
+                            val[e] += e == 0 ? bv[cb].x : e == 1 ? bv[cb].y : e == 2 ? bv[cb].z : bv[cb].w;
+                        if (relu) val[e] = val[e] > 0.0f ? val[e] : 0.0f;
                         const u16 mb = (u16)(m2[e >> 1] >> (16 * (e & 1)));
-                        if (mask && !(from_bf16(mb) > 0.0f)) val = 0.0f;
-                        ov[e] = to_bf16(val);
+                        if (mask && !(from_bf16(mb) > 0.0f)) val[e] = 0.0f;
                     }
                     uint2 packed;
-                    packed.x = (uint32_t)ov[0] | ((uint32_t)ov[1] << 16);
-                    packed.y = (uint32_t)ov[2] | ((uint32_t)ov[3] << 16);
-                    *reinterpret_cast<uint2*>(y + v * ycs + yco + c0) = packed;
+                    packed.x = pack_bf16(val[0], val[1]);
+                    packed.y = pack_bf16(val[2], val[3]);
+                    *reinterpret_cast<uint2*>(yv + cb * 16) = packed;
                 }
             }
         }
@@ -916,7 +1002,9 @@ template <int CIN, int COUT>
 struct ConvTile {
     static constexpr int R = CIN <= 8 ? 4 : (CIN <= 16 ? 2 : 1);
     static constexpr int XW = CIN <= 16 ? 64 : 32;
-    static constexpr size_t LDS = (size_t)3 * (CIN / 8) * (4 * R + 2) * (XW + 2) * 16;
+    static constexpr size_t LDS =
+        conv_slab_bytes(CIN, R, XW) +
+        (conv_weights_in_lds(CIN, COUT, R, XW) ? conv_weight_bytes(CIN, COUT) : 0);
 };
 
 template <int CIN, int COUT>
