@@ -22,12 +22,9 @@
 //
 // Weight gradient: dW[co][tap][ci] = sum_v dY[v][co] X[v + off(tap)][ci],
 // a GEMM reduced over voxels: A = dY (16 co x 32 voxels), B = X shifted by
-// the tap (32 voxels x 16 ci), both read 16 bytes at a time from
-// channel-major, row-padded copies [C][nz][ny][nxp] (three x-shifted copies
-// of X, so every load is aligned). Each work-group reduces a share of the
-// rows for one tap; its waves' sums are combined in LDS in a fixed order and
-// written as a partial; a second kernel sums the partials in a fixed order,
-// so the gradient is deterministic.
+// the tap (32 voxels x 16 ci), both read transposed from slabs in LDS. Each
+// work-group reduces a tile marching in z and writes a partial; a second kernel
+// sums the partials in a fixed order, so the gradient is deterministic.
 #include <initializer_list>
 
 #include "ostr_internal.h"
@@ -457,30 +454,46 @@ __global__ __launch_bounds__(256 + 64 * conv_loaders(conv_slab(CIN, R, XW))) voi
 // (halo included, zero outside the volume) in a 3-slot ring and dY of slice z
 // in a 2-slot ring, both in the convolution's [c8][row][x] layout, the next
 // slices fetched into registers during compute (no global load is waited on
-// inside the step). blockIdx.y picks one 16-channel block of the output
-// (cob) and one share (tg) of its 27 NCI (tap, 16-channel input block)
-// accumulators, which are dealt to the 4 waves round-robin; every wave also
-// sums dY against ones for the bias (share 0's wave 0 keeps it). Each
-// group writes its partial sums: part[g][co][tap CIN + ci], bpart[g][co].
-// Channels past CIN (CIN = 8) read channels 0..7 again; their columns are not
-// written.
+// inside the step). blockIdx.y picks CG of the input channels and CO of the
+// output channels; each group writes its partial sums: part[g][co][tap CIN + ci],
+// bpart[g][co] (the groups of the first input channels).
+//
+// The 9 NCI items (dz, dx, 16-channel input block) are dealt to the 4 waves
+// round-robin. A wave walks the slab's TY + 2 rows; the B operand of item
+// (dz, dx) at slab row y serves the dY rows y - dyi of all three dy and every
+// output block, 3 NCO MFMAs per read pair, with the A operands of the last three
+// dY rows kept in registers (a ring of 4: the next row is read ahead). One read pair per MFMA is twice what LDS delivers
+// per matrix instruction (1 KB per 16 cycles and SIMD), and the rows' reads are
+// issued a step ahead so that a SIMD's only wave does not wait for each.
+// An accumulator still adds its products by (z, row, x). Channels past CIN
+// (CIN = 8) read channels 0..7 again; their columns are not written.
+// One read pair per MFMA in a rolled loop, and now: at 256x256x48 voxels 48->16
+// 326 and 190 us, 16->16 122 and 88, 8->16 111 and 72; at 128x128x24 96->32 203
+// and 104, 32->32 62 and 39, 16->32 29.5 and 27; at 64x64x12 64->64 49 and 41,
+// 32->64 28.5 and 25.
 constexpr int wgrad_xw(int cin) { return cin >= 64 ? 32 : 64; }
 constexpr int wgrad_ty(int cin, int cout) { return cin <= 16 && cout <= 16 ? 8 : 4; }
+// channels of a group: as many as fit its registers (9 ceil(CG / 16) items on 4
+// waves, 3 CO / 16 accumulators each) with the slabs in LDS
+constexpr int wgrad_cg(int cin) { return cin > 48 ? cin / 2 : cin; }
+constexpr int wgrad_co(int cout) { return cout > 32 ? cout / 2 : cout; }
 constexpr int wgrad_slab(int cin, int cout) {
-    return cin / 8 * (wgrad_ty(cin, cout) + 2) * (wgrad_xw(cin) + 2);
+    return wgrad_cg(cin) / 8 * (wgrad_ty(cin, cout) + 2) * (wgrad_xw(cin) + 2);
 }
-constexpr int wgrad_dslab(int cin, int cout) { return 2 * wgrad_ty(cin, cout) * wgrad_xw(cin); }
-// accumulator tiles of one output block, their shares (at most 28 per wave)
-constexpr int wgrad_tiles(int cin) { return 27 * ((cin + 15) / 16); }
-constexpr int wgrad_shares(int cin) { return (wgrad_tiles(cin) + 111) / 112; }
+constexpr int wgrad_dslab(int cin, int cout) {
+    return wgrad_co(cout) / 8 * wgrad_ty(cin, cout) * wgrad_xw(cin);
+}
+constexpr int wgrad_shares(int cin, int cout) {
+    return cin / wgrad_cg(cin) * (cout / wgrad_co(cout));
+}
 
+// the 8 voxels of one operand: two transposing reads, 4 voxels (64 bytes) apart
 typedef short v4i16 __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ bf16x8 tr_read8(const uint4* base, int off0, int off1) {
+__device__ __forceinline__ bf16x8 tr_read8(const __attribute__((address_space(3))) char* b) {
     typedef __attribute__((address_space(3))) v4i16 lds_v4;
-    const char* b = reinterpret_cast<const char*>(base);
     typedef short v8i16 __attribute__((ext_vector_type(8)));
-    const v4i16 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4*)(b + off0));
-    const v4i16 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4*)(b + off1));
+    const v4i16 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4*)b);
+    const v4i16 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4*)(b + 64));
     const v8i16 both = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
     return __builtin_bit_cast(bf16x8, both);
 }
@@ -490,18 +503,19 @@ __global__ __launch_bounds__(256) void wgrad_lds_kernel(
     const u16* __restrict__ x, int xcs, int xco, const u16* __restrict__ dy, int dcs, int dco,
     float* __restrict__ part, float* __restrict__ bpart, int nz, int ny, int nx, int tiles_x,
     int tiles_y, int zc) {
-    constexpr int NC8 = CIN / 8, NCI = (CIN + 15) / 16;
-    constexpr int XW = wgrad_xw(CIN), WG_TY = wgrad_ty(CIN, COUT), KPR = XW / 32;
-    constexpr int TR = WG_TY + 2, TW = XW + 2;
+    constexpr int CG = wgrad_cg(CIN), CO = wgrad_co(COUT);
+    constexpr int NC8 = CG / 8, ND8 = CO / 8, NCI = (CG + 15) / 16, NCO = CO / 16;
+    constexpr int XW = wgrad_xw(CIN), TY = wgrad_ty(CIN, COUT), KPR = XW / 32;
+    constexpr int TR = TY + 2, TW = XW + 2;
     constexpr int SLAB = wgrad_slab(CIN, COUT), DSLAB = wgrad_dslab(CIN, COUT);
-    constexpr int TC = wgrad_tiles(CIN), TG = wgrad_shares(CIN);
-    constexpr int TPW = (TC + TG - 1) / TG;  // tiles per work-group
-    constexpr int NTW = (TPW + 3) / 4;       // tiles per wave
-    extern __shared__ uint4 lds[];           // 3 X slabs, then 2 dY slabs
+    constexpr int NI = 9 * NCI, NIW = (NI + 3) / 4;  // items, items per wave
+    extern __shared__ uint4 lds[];                   // 3 X slabs, then 2 dY slabs
+    typedef __attribute__((address_space(3))) char lds_char;
     uint4* xs = lds;
     uint4* ds = lds + 3 * SLAB;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int cob = (int)blockIdx.y / TG, tg = (int)blockIdx.y % TG;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int co0 = (int)blockIdx.y % (COUT / CO) * CO, ci0 = (int)blockIdx.y / (COUT / CO) * CG;
     const int n_groups = (int)gridDim.x;
     int t;
     {
@@ -512,15 +526,13 @@ __global__ __launch_bounds__(256) void wgrad_lds_kernel(
     const int tx = t % tiles_x;
     t /= tiles_x;
     const int ty = t % tiles_y, tz = t / tiles_y;
-    const int x0 = tx * XW, y0 = ty * WG_TY, z0 = tz * zc;
+    const int x0 = tx * XW, y0 = ty * TY, z0 = tz * zc;
     const int z1 = z0 + zc < nz ? z0 + zc : nz;
-    const int dco_b = dco + 16 * cob;
 
     // This thread's slab elements e = threadIdx.x + 256 i: X slab elements
     // (e < SLAB, [c8][row][x] with the halo) and dY slab elements (SLAB <= e <
-    // SLAB + DSLAB, this group's 16 output channels); their offsets inside a
-    // slice (-1: outside the volume's x/y range, zero) and their LDS index
-    // inside a slot, computed once.
+    // SLAB + DSLAB); their offsets inside a slice (-1: outside the volume's x/y
+    // range, zero) and their LDS index inside a slot, computed once.
     constexpr int NE = (SLAB + DSLAB + 255) / 256;
     int soff[NE], loff[NE];
 #pragma unroll
@@ -533,15 +545,15 @@ __global__ __launch_bounds__(256) void wgrad_lds_kernel(
             const int xi = rest % TW, row = rest / TW;
             const int gx = x0 - 1 + xi, gy = y0 - 1 + row;
             if ((unsigned)gx < (unsigned)nx && (unsigned)gy < (unsigned)ny)
-                soff[i] = (gy * nx + gx) * xcs + xco + c8 * 8;
+                soff[i] = (gy * nx + gx) * xcs + xco + ci0 + c8 * 8;
             loff[i] = (c8 * TR + row) * TW + xi;
         } else if (e < SLAB + DSLAB) {
             const int f = e - SLAB;
-            const int c8 = f & 1, rest = f >> 1;
+            const int c8 = f % ND8, rest = f / ND8;
             const int xi = rest % XW, row = rest / XW;
             const int gx = x0 + xi, gy = y0 + row;
-            if (gx < nx && gy < ny) soff[i] = (gy * nx + gx) * dcs + dco_b + c8 * 8;
-            loff[i] = (c8 * WG_TY + row) * XW + xi;
+            if (gx < nx && gy < ny) soff[i] = (gy * nx + gx) * dcs + dco + co0 + c8 * 8;
+            loff[i] = (c8 * TY + row) * XW + xi;
         }
     }
     const int64_t xslice = (int64_t)ny * nx * xcs, dslice = (int64_t)ny * nx * dcs;
@@ -583,9 +595,29 @@ __global__ __launch_bounds__(256) void wgrad_lds_kernel(
     // group kg addresses channels 4 (s & 3) .. + 3 of voxel 8 kg + (s >> 2)
     const int s = lane & 15, kg = lane >> 4;
     const int pc = (s & 3) >> 1, hb = (s & 1) * 8, vx = 8 * kg + (s >> 2);
-    f32x4 acc[NTW], accb = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    // Byte offset of item i's operand at row 0 inside its slot, and the slot; a
+    // wave's places past the last item repeat it (not written).
+    int item_at[NIW], item_slot[NIW];
 #pragma unroll
-    for (int i = 0; i < NTW; ++i) acc[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int i = 0; i < NIW; ++i) {
+        const int u = wave + 4 * i < NI ? wave + 4 * i : NI - 1;
+        const int dzi = u / (3 * NCI), dxi = u / NCI % 3, cb = u % NCI;
+        const int c8 = 2 * cb + pc < NC8 ? 2 * cb + pc : NC8 - 1;
+        item_at[i] = (c8 * TR * TW + vx + dxi) * 16 + hb;
+        item_slot[i] = (z0 + dzi + 2) % 3;
+    }
+    const int dy_at = (pc * TY * XW + vx) * 16 + hb;
+    const lds_char* const xl = (const lds_char*)xs;
+    const lds_char* const dl = (const lds_char*)ds;
+    f32x4 acc[NIW][3][NCO], accb[NCO];
+#pragma unroll
+    for (int c = 0; c < NCO; ++c) {
+        accb[c] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int i = 0; i < NIW; ++i)
+#pragma unroll
+            for (int d = 0; d < 3; ++d) acc[i][d][c] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    }
     bf16x8 ones;
 #pragma unroll
     for (int e = 0; e < 8; ++e) ones[e] = (__bf16)1.0f;
@@ -593,29 +625,44 @@ __global__ __launch_bounds__(256) void wgrad_lds_kernel(
     for (int z = z0; z < z1; ++z) {
         const bool more = z + 1 < z1;
         if (more) fetch(z + 2, z + 1);
-        const uint4* dslot = ds + ((z + 2) % 2) * DSLAB;
-#pragma unroll 1
-        for (int kc = 0; kc < KPR * WG_TY; ++kc) {
-            const int r = kc / KPR, xh = (kc % KPR) * 32;
-            // A: dY of voxels (x0 + xh + 8 kg .. + 7, row r), channels 16 cob .. + 15
-            const int aoff = ((pc * WG_TY + r) * XW + xh + vx) * 16 + hb;
-            const bf16x8 a = tr_read8(dslot, aoff, aoff + 4 * 16);
-            // branch-free, so that the reads of all tiles can be issued ahead:
-            // every wave sums the bias, and a wave's slots past its share's
-            // last tile repeat a tile (not written)
-            accb = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, ones, accb, 0, 0, 0);
+        const lds_char* pb[NIW];
 #pragma unroll
-            for (int i = 0; i < NTW; ++i) {
-                const int ul = wave + 4 * i < TPW ? wave + 4 * i : TPW - 1;
-                const int u = tg * TPW + ul < TC ? tg * TPW + ul : TC - 1;
-                const int tap = u / NCI, cb = u % NCI;
-                const int dzi = tap / 9, dyi = (tap / 3) % 3, dxi = tap % 3;
-                const int c8 = 2 * cb + pc < NC8 ? 2 * cb + pc : NC8 - 1;
-                const uint4* xslot = xs + ((z + dzi + 2) % 3) * SLAB;
-                const int boff = ((c8 * TR + r + dyi) * TW + xh + vx + dxi) * 16 + hb;
-                const bf16x8 b = tr_read8(xslot, boff, boff + 4 * 16);
-                acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc[i], 0, 0, 0);
-            }
+        for (int i = 0; i < NIW; ++i) {
+            pb[i] = xl + item_slot[i] * (SLAB * 16) + item_at[i];
+            item_slot[i] = item_slot[i] == 2 ? 0 : item_slot[i] + 1;
+        }
+        const lds_char* const pa = dl + ((z + 2) % 2) * (DSLAB * 16) + dy_at;
+        bf16x8 a[4][KPR][NCO], b[2][NIW];
+        auto read_step = [&](int st) {  // step st: slab row st / KPR, columns 32 (st % KPR) ..
+            const int r = st / KPR, h = st % KPR;
+#pragma unroll
+            for (int c = 0; c < NCO; ++c)
+                if (r < TY) a[r % 4][h][c] = tr_read8(pa + ((2 * c * TY + r) * XW + 32 * h) * 16);
+#pragma unroll
+            for (int i = 0; i < NIW; ++i) b[st % 2][i] = tr_read8(pb[i] + (r * TW + 32 * h) * 16);
+        };
+        read_step(0);
+#pragma unroll
+        for (int st = 0; st < TR * KPR; ++st) {
+            const int r = st / KPR, h = st % KPR;
+            if (st + 1 < TR * KPR) read_step(st + 1);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int c = 0; c < NCO; ++c)
+                if (r < TY)
+                    accb[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[r % 4][h][c], ones, accb[c],
+                                                                      0, 0, 0);
+#pragma unroll
+            for (int i = 0; i < NIW; ++i)
+#pragma unroll
+                for (int d = 0; d < 3; ++d) {
+                    if (r - d < 0 || r - d >= TY) continue;
+#pragma unroll
+                    for (int c = 0; c < NCO; ++c)
+                        acc[i][d][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                            a[(r - d) % 4][h][c], b[st % 2][i], acc[i][d][c], 0, 0, 0);
+                }
+            __builtin_amdgcn_sched_barrier(0);
         }
         if (more) {
             __syncthreads();  // slice z - 1's X slot and dY slot are read no more
@@ -623,23 +670,30 @@ __global__ __launch_bounds__(256) void wgrad_lds_kernel(
             __syncthreads();
         }
     }
-    // D row co = 16 cob + 4 kg + e, column ci = lane & 15
+    // D row co = co0 + 16 c + 4 kg + e, column ci = ci0 + 16 cb + (lane & 15)
     constexpr int K = 27 * CIN;
-    float* out = part + (int64_t)group * COUT * K;
+    float* out = part + (int64_t)group * COUT * K + (int64_t)(co0 + 4 * kg) * K;
 #pragma unroll
-    for (int i = 0; i < NTW; ++i) {
-        const int ul = wave + 4 * i, u = tg * TPW + ul;
-        if (ul >= TPW || u >= TC) continue;
-        const int tap = u / NCI, ci = (u % NCI) * 16 + (lane & 15);
-        if (ci < CIN) {
+    for (int i = 0; i < NIW; ++i) {
+        const int u = wave + 4 * i;
+        if (u >= NI) continue;
+        const int dzi = u / (3 * NCI), dxi = u / NCI % 3, ci = (u % NCI) * 16 + (lane & 15);
+        if (ci >= CG) continue;
+#pragma unroll
+        for (int d = 0; d < 3; ++d)
+#pragma unroll
+            for (int c = 0; c < NCO; ++c)
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    out[(int64_t)(16 * c + e) * K + (dzi * 9 + d * 3 + dxi) * CIN + ci0 + ci] =
+                        acc[i][d][c][e];
+    }
+    if (ci0 == 0 && wave == 0 && (lane & 15) == 0) {
+#pragma unroll
+        for (int c = 0; c < NCO; ++c)
 #pragma unroll
             for (int e = 0; e < 4; ++e)
-                out[(int64_t)(16 * cob + 4 * kg + e) * K + tap * CIN + ci] = acc[i][e];
-        }
-    }
-    if (tg == 0 && wave == 0 && (lane & 15) == 0) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) bpart[(int64_t)group * COUT + 16 * cob + 4 * kg + e] = accb[e];
+                bpart[(int64_t)group * COUT + co0 + 16 * c + 4 * kg + e] = accb[c][e];
     }
 }
 
@@ -1128,7 +1182,7 @@ static hipError_t wgrad_lds_t(const void* x, int xcs, int xco, const void* dy, i
             (const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) return e;
     }
-    const dim3 grid((unsigned)g.groups, (unsigned)(COUT / 16 * wgrad_shares(CIN)));
+    const dim3 grid((unsigned)g.groups, (unsigned)wgrad_shares(CIN, COUT));
     hipLaunchKernelGGL(kern, grid, dim3(256), lds, st, (const u16*)x, xcs, xco, (const u16*)dy,
                        dcs, dco, part, bpart, nz, ny, nx, g.tiles_x, g.tiles_y, g.zc);
     hipLaunchKernelGGL(sum_parts_kernel, dim3(sum_parts_grid(n)), dim3(256), 0, st,
