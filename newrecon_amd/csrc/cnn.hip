@@ -80,9 +80,15 @@ __device__ __forceinline__ bf16x8 zero8() {
 // loads wait for the step before's stores, see the epilogue). At 256x256x48
 // voxels, weights per chunk and in LDS: 16->48 345 and 270 us, 16->32 33 and 27
 // (128x128x24), 32->32 72 and 42, 32->64 25 and 16 (64x64x12).
+// Weights read per chunk come from L2, 3 KB per output block and wave: there a
+// wave takes twice the rows and half the output channels, so that the group reads
+// them twice and not four times, and they are asked for two chunks ahead, or
+// eight where registers allow, instead of one. All channels and one chunk, then
+// half and two or eight: 96->32 190 and 136 us, 32->96 180 and 120 (128x128x24),
+// 64->64 59 and 36, 64->32 31 and 22 (64x64x12).
 // Slab elements per LDS slot, and loader waves: each holds at most 24 of its
 // 16-byte elements per lane in flight.
-constexpr int conv_slab(int cin, int r, int xw) { return cin / 8 * (4 * r + 2) * (xw + 2); }
+constexpr int conv_slab(int cin, int rows, int xw) { return cin / 8 * (rows + 2) * (xw + 2); }
 constexpr int conv_loaders(int slab) { return (slab + 64 * 24 - 1) / (64 * 24); }
 
 // Weights of a wave in registers (the rule and its budget are in the kernel),
@@ -93,22 +99,32 @@ constexpr bool conv_weights_in_registers(int cin, int cout, int r, int xw) {
     const int acc = 4 * r * (xw / 16) * (cout / 16) + (pipe ? 4 * (r + 2) * (xw / 16) : 0);
     return 12 * conv_chunks(cin) * (cout / 16) + acc <= (pipe ? 220 : 180);
 }
-constexpr int conv_slab_bytes(int cin, int r, int xw) { return (3 * conv_slab(cin, r, xw) + 64) * 16; }
+constexpr int conv_slab_bytes(int cin, int rows, int xw) {
+    return (3 * conv_slab(cin, rows, xw) + 64) * 16;
+}
 constexpr int conv_weight_bytes(int cin, int cout) { return conv_chunks(cin) * 3 * (cout / 16) * 1024; }
 constexpr bool conv_weights_in_lds(int cin, int cout, int r, int xw) {
     return !conv_weights_in_registers(cin, cout, r, xw) &&
-           conv_slab_bytes(cin, r, xw) + conv_weight_bytes(cin, cout) <= 160 * 1024;
+           conv_slab_bytes(cin, 4 * r, xw) + conv_weight_bytes(cin, cout) <= 160 * 1024;
+}
+// Output-channel halves (2) or all channels in each wave (1); see ConvTile.
+constexpr int conv_co_split(int cin, int cout, int r, int xw) {
+    return !conv_weights_in_registers(cin, cout, r, xw) &&
+                   !conv_weights_in_lds(cin, cout, r, xw) && cout % 32 == 0
+               ? 2
+               : 1;
 }
 
-template <int CIN, int COUT, int R, int XW>
-__global__ __launch_bounds__(256 + 64 * conv_loaders(conv_slab(CIN, R, XW))) void conv3d_lds_kernel(
+template <int CIN, int COUT, int TY, int XW>
+__global__ __launch_bounds__(256 + 64 * conv_loaders(conv_slab(CIN, TY, XW))) void conv3d_lds_kernel(
     const u16* __restrict__ x, int xcs, int xco, const u16* __restrict__ w,
     const float* __restrict__ bias, u16* __restrict__ y, int ycs, int yco,
     const u16* __restrict__ mask, int mcs, int mco, int relu, int nz, int ny, int nx,
     int tiles_x, int tiles_y, int zc) {
     constexpr int NC8 = CIN / 8, NP = 9 * NC8, NQ = (NP + 3) / 4;
-    constexpr int KP = kpad(CIN), NCO = COUT / 16, NVB = XW / 16;
-    constexpr int TR = 4 * R + 2, TW = XW + 2, SLAB = conv_slab(CIN, R, XW);
+    constexpr int CS = conv_co_split(CIN, COUT, TY / 4, XW), R = CS * TY / 4;
+    constexpr int KP = kpad(CIN), NCO = COUT / 16 / CS, NVB = XW / 16;
+    constexpr int TR = TY + 2, TW = XW + 2, SLAB = conv_slab(CIN, TY, XW);
     constexpr int LW = conv_loaders(SLAB), NT = 256 + 64 * LW;
     extern __shared__ uint4 slabs[];  // 3 * SLAB, then one place per lane
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -124,8 +140,9 @@ __global__ __launch_bounds__(256 + 64 * conv_loaders(conv_slab(CIN, R, XW))) voi
     const int tx = t % tiles_x;
     t /= tiles_x;
     const int ty = t % tiles_y, tz = t / tiles_y;
-    const int x0 = tx * XW, y0 = ty * 4 * R, z0 = tz * zc;
+    const int x0 = tx * XW, y0 = ty * TY, z0 = tz * zc;
     const int z1 = z0 + zc < nz ? z0 + zc : nz;
+    const int row0 = wave / CS * R, co0 = wave % CS * (16 * NCO);  // of a compute wave
 
     // Slab element e -> (row, xi, c8), c8 fastest (contiguous global reads): its
     // offset inside a slice of x, in 16-byte units, and its place in an LDS
@@ -156,14 +173,14 @@ __global__ __launch_bounds__(256 + 64 * conv_loaders(conv_slab(CIN, R, XW))) voi
         for (int dyi = 0; dyi < 3; ++dyi)
 #pragma unroll
             for (int cb = 0; cb < NCO; ++cb)
-                a[dyi][cb] = p < NP ? load8(w + (int64_t)(cb * 16 + n) * KP +
+                a[dyi][cb] = p < NP ? load8(w + (int64_t)(co0 + cb * 16 + n) * KP +
                                             (dzi * 9 + dyi * 3 + dxi) * CIN + c8 * 8)
                                     : zero8();
     };
     // Weights in LDS as the operands' register image, [q][dyi][cb][lane], each
     // read 1 KB of consecutive 16-byte elements; written by all waves, read
     // after the barrier below.
-    constexpr bool WLDS = conv_weights_in_lds(CIN, COUT, R, XW);
+    constexpr bool WLDS = CS == 1 && conv_weights_in_lds(CIN, COUT, R, XW);
     bf16x8* wl = reinterpret_cast<bf16x8*>(slabs + 3 * SLAB + 64);
     if constexpr (WLDS) {
 #pragma unroll 1
@@ -257,7 +274,7 @@ __global__ __launch_bounds__(256 + 64 * conv_loaders(conv_slab(CIN, R, XW))) voi
         const int c8 = p % NC8, dxi = (p / NC8) % 3, dzi = p / (3 * NC8);
         const int m = (z + 2) % 3;  // slot of slice z - 1
         const int s0 = m * SLAB, s1 = (m == 2 ? 0 : m + 1) * SLAB, s2 = (m == 0 ? 2 : m - 1) * SLAB;
-        return slabs + (dzi == 0 ? s0 : dzi == 1 ? s1 : s2) + (c8 * TR + wave * R) * TW + n + dxi;
+        return slabs + (dzi == 0 ? s0 : dzi == 1 ? s1 : s2) + (c8 * TR + row0) * TW + n + dxi;
     };
     bf16x8 ring[PIPE ? RR : 1][NVB];
     auto read_row = [&](const uint4* bp, int r, bf16x8 (&dst)[NVB]) {
@@ -328,14 +345,20 @@ __global__ __launch_bounds__(256 + 64 * conv_loaders(conv_slab(CIN, R, XW))) voi
     // schedules the reads: conv_weights_in_registers); otherwise each chunk's
     // are read one chunk ahead, or at the chunk where two chunks' would not fit.
     constexpr int ACC = 4 * R * NVB * NCO + (PIPE ? 4 * RR * NVB : 0);
-    constexpr bool AREG = conv_weights_in_registers(CIN, COUT, R, XW);
-    constexpr int NQR = AREG ? NQ : 1, NQA = AREG || 24 * NCO + ACC > 200 ? 1 : 2;
+    constexpr bool AREG = CS == 1 && conv_weights_in_registers(CIN, COUT, R, XW);
+    constexpr int NQR = AREG ? NQ : 1;
+    constexpr int NQA = AREG                                                  ? 1
+                        : !WLDS && NQ % 9 == 0 && 108 * NCO + ACC <= 200      ? 9
+                        : !WLDS && NQ % 3 == 0 && 36 * NCO + ACC <= 200       ? 3
+                        : 24 * NCO + ACC <= 200                               ? 2
+                                                                              : 1;
     bf16x8 aw[NQR][3][NCO], ab[NQA][3][NCO];
     if constexpr (AREG) {
 #pragma unroll
         for (int q = 0; q < NQ; ++q) load_a(q, aw[q]);
-    } else if constexpr (NQA == 2) {
-        operands(0, ab[0]);
+    } else {
+#pragma unroll
+        for (int d = 0; d + 1 < NQA; ++d) operands(d, ab[d]);
     }
     // A wave's memory counter is in order and counts stores: a load asked for
     // in the epilogue would wait for the step before's stores to reach memory.
@@ -347,16 +370,16 @@ __global__ __launch_bounds__(256 + 64 * conv_loaders(conv_slab(CIN, R, XW))) voi
     float4 bv[NCO];
 #pragma unroll
     for (int cb = 0; cb < NCO; ++cb)
-        bv[cb] = bias ? *reinterpret_cast<const float4*>(bias + cb * 16 + kg * 4)
+        bv[cb] = bias ? *reinterpret_cast<const float4*>(bias + co0 + cb * 16 + kg * 4)
                       : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
 #pragma unroll 1
     for (int z = z0; z < z1; ++z) {
         // voxel (x0 + n, first row) of this lane; the others lie a wave-uniform
         // number of voxels on
-        const int gx0 = x0 + n, gy0 = y0 + wave * R;
+        const int gx0 = x0 + n, gy0 = y0 + row0;
         const int64_t v0 = ((int64_t)z * ny + gy0) * nx + gx0;
-        u16* yp = y + v0 * ycs + yco + kg * 4;
-        const u16* mp = mask + v0 * mcs + mco + kg * 4;
+        u16* yp = y + v0 * ycs + yco + co0 + kg * 4;
+        const u16* mp = mask + v0 * mcs + mco + co0 + kg * 4;
         uint2 mk[R][NVB][NCO];
         auto load_masks = [&] {
 #pragma unroll
@@ -387,6 +410,18 @@ __global__ __launch_bounds__(256 + 64 * conv_loaders(conv_slab(CIN, R, XW))) voi
         if constexpr (AREG) {
 #pragma unroll
             for (int q = 0; q < NQ; ++q) chunk(z, q, bq, aw[q], acc);
+        } else if constexpr (NQA > 2) {
+            // the chunk NQA - 1 on is loaded before this one's MFMAs (after the
+            // last chunks: the next slice's first)
+#pragma unroll 1
+            for (int q0 = 0; q0 < NQ; q0 += NQA)
+#pragma unroll
+                for (int d = 0; d < NQA; ++d) {
+                    const int ahead = q0 + d + NQA - 1;
+                    operands(ahead < NQ ? ahead : ahead - NQ, ab[(d + NQA - 1) % NQA]);
+                    __builtin_amdgcn_sched_barrier(0);
+                    chunk(z, q0 + d, bq, ab[d], acc);
+                }
         } else {
 #pragma unroll 1
             for (int q = 0; q < NQ; ++q) {
@@ -1069,13 +1104,13 @@ unsigned grid_for(int64_t n, int per = 256) {
     return (unsigned)(g < 1 ? 1 : g);
 }
 
-// Tile of the LDS convolution: R output rows per wave, XW voxels along x.
+// Tile of the LDS convolution: TY rows by XW voxels along x.
 template <int CIN, int COUT>
 struct ConvTile {
     static constexpr int R = CIN <= 8 ? 4 : (CIN <= 16 ? 2 : 1);
-    static constexpr int XW = CIN <= 16 ? 64 : 32;
+    static constexpr int TY = 4 * R, XW = CIN <= 16 ? 64 : 32;
     static constexpr size_t LDS =
-        conv_slab_bytes(CIN, R, XW) +
+        conv_slab_bytes(CIN, TY, XW) +
         (conv_weights_in_lds(CIN, COUT, R, XW) ? conv_weight_bytes(CIN, COUT) : 0);
 };
 
@@ -1084,14 +1119,14 @@ hipError_t conv_t(const u16* x, int xcs, int xco, const u16* w, const float* bia
                   int ycs, int yco, const u16* mask, int mcs, int mco, int relu, int nz, int ny,
                   int nx, hipStream_t st) {
     using T = ConvTile<CIN, COUT>;
-    const auto kern = conv3d_lds_kernel<CIN, COUT, T::R, T::XW>;
+    const auto kern = conv3d_lds_kernel<CIN, COUT, T::TY, T::XW>;
     if (T::LDS > 65536) {
         const hipError_t e = hipFuncSetAttribute((const void*)kern,
                                                  hipFuncAttributeMaxDynamicSharedMemorySize,
                                                  (int)T::LDS);
         if (e != hipSuccess) return e;
     }
-    const int tiles_x = (nx + T::XW - 1) / T::XW, tiles_y = (ny + 4 * T::R - 1) / (4 * T::R);
+    const int tiles_x = (nx + T::XW - 1) / T::XW, tiles_y = (ny + T::TY - 1) / T::TY;
     // about 256 groups (one per CU): z chunks of zc slices, each with a
     // three-slab prologue; longer chunks measured faster at the training size
     const int64_t tiles = (int64_t)tiles_x * tiles_y;
@@ -1099,7 +1134,7 @@ hipError_t conv_t(const u16* x, int xcs, int xco, const u16* w, const float* bia
     if (nzc > nz) nzc = nz;
     const int zc = (int)((nz + nzc - 1) / nzc);
     nzc = (nz + zc - 1) / zc;
-    const int nt = 256 + 64 * conv_loaders(conv_slab(CIN, T::R, T::XW));
+    const int nt = 256 + 64 * conv_loaders(conv_slab(CIN, T::TY, T::XW));
     hipLaunchKernelGGL(kern, dim3((unsigned)(tiles * nzc)), dim3(nt), T::LDS, st, x, xcs,
                        xco, w, bias, y, ycs, yco, mask, mcs, mco, relu, nz, ny, nx, tiles_x,
                        tiles_y, zc);

@@ -34,7 +34,7 @@ def conv(dev, cin, cout, x, w, bias, mask, relu, stride, offset):
 
 
 @pytest.mark.parametrize("cin,cout", [(8, 16), (16, 16), (16, 32), (32, 32), (32, 64), (96, 32),
-                                      (16, 48)])
+                                      (16, 48), (64, 64), (64, 32), (32, 96)])
 @pytest.mark.parametrize("shape", [(1, 5, 70), (3, 9, 33), (13, 17, 65)])
 def test_ragged_tiles(dev, cin, cout, shape):
     gen = torch.Generator(device=dev).manual_seed(cin * cout + shape[0])
