@@ -734,13 +734,19 @@ __global__ __launch_bounds__(256) void wgrad_lds_kernel(
 
 // dw[i] = sum_s part[s][i], i < n, in a fixed order: four lanes per output
 // sum s = g, g + 4, ... (g = 0..3, s ascending), then (((g0 + g1) + g2) + g3).
-// A work-group covers 64 outputs (grid: ceil(n / 64) groups of 256).
-__global__ __launch_bounds__(256) void sum_parts_kernel(const float* __restrict__ part,
-                                                        int nsplit, int64_t n,
-                                                        float* __restrict__ dw) {
+// A work-group covers 64 outputs; the groups from dw_groups on do the same for
+// the bias (bpart, db, nb), whose launch of its own took 4.8 us.
+__global__ __launch_bounds__(256) void sum_parts_kernel(const float* __restrict__ wpart,
+                                                        int nsplit, int64_t nw,
+                                                        float* __restrict__ dw, int dw_groups,
+                                                        const float* __restrict__ bpart,
+                                                        int64_t nb, float* __restrict__ db) {
     __shared__ float red[4][64];
     const int il = threadIdx.x & 63, g = threadIdx.x >> 6;
-    const int64_t i = (int64_t)blockIdx.x * 64 + il;
+    const bool bias = (int)blockIdx.x >= dw_groups;
+    const float* part = bias ? bpart : wpart;
+    const int64_t n = bias ? nb : nw;
+    const int64_t i = (int64_t)((int)blockIdx.x - (bias ? dw_groups : 0)) * 64 + il;
     float s = 0.0f;
     if (i < n) {
         // eight partials loaded before they are added (in the same order),
@@ -757,7 +763,7 @@ __global__ __launch_bounds__(256) void sum_parts_kernel(const float* __restrict_
     }
     red[g][il] = s;
     __syncthreads();
-    if (g == 0 && i < n) dw[i] = ((red[0][il] + red[1][il]) + red[2][il]) + red[3][il];
+    if (g == 0 && i < n) (bias ? db : dw)[i] = ((red[0][il] + red[1][il]) + red[2][il]) + red[3][il];
 }
 static unsigned sum_parts_grid(int64_t n) { return (unsigned)((n + 63) / 64); }
 
@@ -1220,11 +1226,9 @@ static hipError_t wgrad_lds_t(const void* x, int xcs, int xco, const void* dy, i
     const dim3 grid((unsigned)g.groups, (unsigned)wgrad_shares(CIN, COUT));
     hipLaunchKernelGGL(kern, grid, dim3(256), lds, st, (const u16*)x, xcs, xco, (const u16*)dy,
                        dcs, dco, part, bpart, nz, ny, nx, g.tiles_x, g.tiles_y, g.zc);
-    hipLaunchKernelGGL(sum_parts_kernel, dim3(sum_parts_grid(n)), dim3(256), 0, st,
-                       (const float*)part, g.groups, n, dw);
-    if (db)
-        hipLaunchKernelGGL(sum_parts_kernel, dim3(sum_parts_grid(COUT)), dim3(256), 0, st,
-                           (const float*)bpart, g.groups, (int64_t)COUT, db);
+    const unsigned gw = sum_parts_grid(n), gb = db ? sum_parts_grid(COUT) : 0;
+    hipLaunchKernelGGL(sum_parts_kernel, dim3(gw + gb), dim3(256), 0, st, (const float*)part,
+                       g.groups, n, dw, (int)gw, (const float*)bpart, (int64_t)COUT, db);
     return hipGetLastError();
 }
 
