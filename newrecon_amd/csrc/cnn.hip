@@ -1120,6 +1120,24 @@ struct ConvTile {
         (conv_weights_in_lds(CIN, COUT, R, XW) ? conv_weight_bytes(CIN, COUT) : 0);
 };
 
+// Slices per group: the z chunking with the least (groups on the busiest of 256
+// CUs) x (slices + 2), two for the prologue's slabs. As many chunks as made at
+// least 256 groups left 4 to 24 CUs with twice the others' work where the tiles do
+// not divide 256 (260 groups at 200x100x20: 16->16 35 us, now 24 with 208; 96->32 at
+// 100x50x10 52 and 40, 8->16 27 and 21, 32->32 20 and 16, 48->16 53 and 49); where
+// they do (256x256x48 and its halves) the chunks are the same.
+static int conv_chunk(int64_t tiles, int nz) {
+    int best = nz;
+    int64_t best_cost = INT64_MAX;
+    for (int nzc = 1; nzc <= nz && (nzc == 1 || tiles * nzc <= 4096); ++nzc) {
+        const int zc = (nz + nzc - 1) / nzc;
+        const int64_t rounds = (tiles * ((nz + zc - 1) / zc) + 255) / 256;
+        const int64_t cost = rounds * (zc + 2);
+        if (cost < best_cost) best = zc, best_cost = cost;
+    }
+    return best;
+}
+
 template <int CIN, int COUT>
 hipError_t conv_t(const u16* x, int xcs, int xco, const u16* w, const float* bias, u16* y,
                   int ycs, int yco, const u16* mask, int mcs, int mco, int relu, int nz, int ny,
@@ -1133,13 +1151,10 @@ hipError_t conv_t(const u16* x, int xcs, int xco, const u16* w, const float* bia
         if (e != hipSuccess) return e;
     }
     const int tiles_x = (nx + T::XW - 1) / T::XW, tiles_y = (ny + T::TY - 1) / T::TY;
-    // about 256 groups (one per CU): z chunks of zc slices, each with a
-    // three-slab prologue; longer chunks measured faster at the training size
+    // z chunks of zc slices, each with a three-slab prologue
     const int64_t tiles = (int64_t)tiles_x * tiles_y;
-    int64_t nzc = (256 + tiles - 1) / tiles;
-    if (nzc > nz) nzc = nz;
-    const int zc = (int)((nz + nzc - 1) / nzc);
-    nzc = (nz + zc - 1) / zc;
+    const int zc = conv_chunk(tiles, nz);
+    const int64_t nzc = (nz + zc - 1) / zc;
     const int nt = 256 + 64 * conv_loaders(conv_slab(CIN, T::TY, T::XW));
     hipLaunchKernelGGL(kern, dim3((unsigned)(tiles * nzc)), dim3(nt), T::LDS, st, x, xcs,
                        xco, w, bias, y, ycs, yco, mask, mcs, mco, relu, nz, ny, nx, tiles_x,
