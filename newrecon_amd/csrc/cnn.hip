@@ -1015,31 +1015,33 @@ __global__ __launch_bounds__(256) void output_smooth_kernel(
     constexpr int PAD = 2 * CNN_SMOOTH_MAX_R, H = SMOOTH_Y + PAD, W = SMOOTH_X + PAD;
     __shared__ float val[H][W], row[H][SMOOTH_X];
     const int tiles_x = (nx + SMOOTH_X - 1) / SMOOTH_X, tiles_y = (ny + SMOOTH_Y - 1) / SMOOTH_Y;
-    const int t = blockIdx.x;
-    const int x0 = (t % tiles_x) * SMOOTH_X, y0 = (t / tiles_x) % tiles_y * SMOOTH_Y;
-    const int64_t plane = (int64_t)(t / tiles_x / tiles_y) * ny * nx;
+    const int64_t tiles = (int64_t)tiles_x * tiles_y * nz;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int h = SMOOTH_Y + 2 * r, w = SMOOTH_X + 2 * r;
-    for (int e = threadIdx.x; e < h * w; e += 256) {
-        const int j = e / w, i = e - j * w;
-        const int yy = min(max(y0 + j - r, 0), ny - 1), xx = min(max(x0 + i - r, 0), nx - 1);
-        val[j][i] = from_bf16(out[(plane + (int64_t)yy * nx + xx) * ocs]);
-    }
-    __syncthreads();
-    for (int j = wave; j < h; j += 4) {
-        float s = 0.0f;
-        for (int i = 0; i <= 2 * r; ++i) s = fmaf(T.w[i], val[j][lane + i], s);
-        row[j][lane] = s;
-    }
-    __syncthreads();
-    const int x = x0 + lane;
-    if (x >= nx) return;
-    for (int k = wave; k < SMOOTH_Y && y0 + k < ny; k += 4) {
-        float acc = 0.0f;
-        for (int j = 0; j <= 2 * r; ++j) acc = fmaf(T.w[j], row[k + j][lane], acc);
-        const int64_t v = plane + (int64_t)(y0 + k) * nx + x;
-        const float p = img[v] + acc * inv_scale;
-        pred[v] = (clamp && p < 0.0f) ? 0.0f : p;
+    for (int64_t t = blockIdx.x; t < tiles; t += gridDim.x) {
+        const int x0 = (int)(t % tiles_x) * SMOOTH_X, y0 = (int)(t / tiles_x % tiles_y) * SMOOTH_Y;
+        const int64_t plane = t / tiles_x / tiles_y * ny * nx;
+        for (int e = threadIdx.x; e < h * w; e += 256) {
+            const int j = e / w, i = e - j * w;
+            const int yy = min(max(y0 + j - r, 0), ny - 1), xx = min(max(x0 + i - r, 0), nx - 1);
+            val[j][i] = from_bf16(out[(plane + (int64_t)yy * nx + xx) * ocs]);
+        }
+        __syncthreads();
+        for (int j = wave; j < h; j += 4) {
+            float s = 0.0f;
+            for (int i = 0; i <= 2 * r; ++i) s = fmaf(T.w[i], val[j][lane + i], s);
+            row[j][lane] = s;
+        }
+        __syncthreads();  // the row sums are complete, the values read no more
+        const int x = x0 + lane;
+        for (int k = wave; x < nx && k < SMOOTH_Y && y0 + k < ny; k += 4) {
+            float acc = 0.0f;
+            for (int j = 0; j <= 2 * r; ++j) acc = fmaf(T.w[j], row[k + j][lane], acc);
+            const int64_t v = plane + (int64_t)(y0 + k) * nx + x;
+            const float p = img[v] + acc * inv_scale;
+            pred[v] = (clamp && p < 0.0f) ? 0.0f : p;
+        }
+        // the next tile's row sums come after its first barrier, past every read here
     }
 }
 
@@ -1352,8 +1354,7 @@ hipError_t launch_cnn_output_smooth(const void* out, int ocs, const float* img, 
     for (int k = 0; k <= 2 * r; ++k) T.w[k] = taps[k];
     const int64_t tiles = (int64_t)((nx + SMOOTH_X - 1) / SMOOTH_X) *
                           ((ny + SMOOTH_Y - 1) / SMOOTH_Y) * nz;
-    if (tiles > 0x7fffffff) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(output_smooth_kernel, dim3((unsigned)tiles), dim3(256), 0, st,
+    hipLaunchKernelGGL(output_smooth_kernel, dim3(grid_for(tiles, 1)), dim3(256), 0, st,
                        (const u16*)out, ocs, img, nz, ny, nx, inv_scale, T, r, clamp, pred);
     return hipGetLastError();
 }

@@ -1,5 +1,5 @@
 """The smoothed residual of the network (ostr_cnn_output_smooth) on slices that cut its
-tiles raggedly, smaller than the filter and of several slices, for every radius: against
+tiles raggedly, smaller than the filter, of several slices and of more slices than groups, for every radius: against
 the FP64 filter with repeated edges. Two sums of 2r + 1 FP32 FMAs with taps that sum to
 1 err by at most 2 (2r + 1) half-ulps of the largest value, and three more roundings
 follow: (4 r + 5) * 2^-24 of the peak."""
@@ -15,7 +15,8 @@ from newrecon_amd.warmstart import _ptr, cnn_lib
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("shape", [(1, 1, 4), (2, 3, 2), (1, 16, 64), (3, 17, 65), (2, 50, 131)])
+@pytest.mark.parametrize("shape", [(1, 1, 4), (2, 3, 2), (1, 16, 64), (3, 17, 65), (2, 50, 131),
+                                   (65540, 1, 2)])
 @pytest.mark.parametrize("r", [0, 1, 3, 4])
 @pytest.mark.parametrize("ocs,clamp", [(16, 0), (8, 1)])
 def test_tiles_and_edges(dev, shape, r, ocs, clamp):
