@@ -41,7 +41,7 @@ def algorithmic_bytes(geom, vs, kernel, s_img=4, s_prj=4):
 PROFILE_JSON = os.path.join(ROOT, "profiles",
                             "fproj_h-update_fused_dbt-clinical-1400x600x60-15v.json")
 PROFILED_KERNEL = {"fproj_h": "project_kernel<3, float, float>",
-                   "update_fused": "update_fused_kernel<2, float, float>"}
+                   "update_fused": "update_fused_kernel<2, float, float, 8>"}
 
 
 VALU_JSON = os.path.join(ROOT, "profiles",

@@ -33,7 +33,7 @@ CALIB_KIB = 262144.0  # 256 MiB
 
 
 def short_name(name: str) -> str:
-    m = re.search(r"ostr::\(anonymous namespace\)::(\w+)(<[^(]*>)?", name)
+    m = re.search(r"ostr::(?:\(anonymous namespace\)::)?(\w+)(<[^(]*>)?", name)
     if m:
         return m.group(1) + (m.group(2) or "")
     return name.split("(")[0][:60]
