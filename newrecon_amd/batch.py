@@ -44,8 +44,10 @@ class TileCfg(ctypes.Structure):
         return f"TileCfg({self.as_dict()})"
 
 
-# the single-case kernels' shapes: 64x4 bins, 64x(8x4) voxels, one group per tile
-DEFAULT_TILE = dict(fwd_rows=4, fwd_groups_per_cu=0, upd_rows=8, upd_waves=4,
+# 64x1 bins, 64x(8x2) voxels, one group per tile: small groups leave no wave's
+# registers waiting for the rest of its group (four uneven cases, one step each:
+# 64x4 bins and 4 waves 551 us, 2 waves 538, 64x1 bins too 533)
+DEFAULT_TILE = dict(fwd_rows=1, fwd_groups_per_cu=0, upd_rows=8, upd_waves=2,
                     upd_groups_per_cu=0)
 
 

@@ -16,7 +16,7 @@ namespace ostr {
 namespace {
 
 template <typename TP, int R>
-__global__ __launch_bounds__(256) void sbp_kernel(DevGeom g, SlotTab S, int n_slots,
+__global__ __launch_bounds__(64 * CASE_WAVES) void sbp_kernel(DevGeom g, SlotTab S, int n_slots,
                                                   const TP* __restrict__ prj,
                                                   float* __restrict__ img) {
     const TileCoord c = tile_coord<R, CASE_WAVES>(g, xcd_tile(blockIdx.x, gridDim.x));
@@ -43,7 +43,7 @@ __global__ __launch_bounds__(256) void sbp_kernel(DevGeom g, SlotTab S, int n_sl
 //   x = max(0, x + lambda * (u + beta * prior / sens))  (PRIOR true; the sign is
 //                                                        the reference's)
 template <typename TP, bool PRIOR, int R>
-__global__ __launch_bounds__(256) void sart_update_kernel(DevGeom g, SlotTab S, int n_slots,
+__global__ __launch_bounds__(64 * CASE_WAVES) void sart_update_kernel(DevGeom g, SlotTab S, int n_slots,
                                                           const TP* __restrict__ diff,
                                                           float* __restrict__ img,
                                                           const float* __restrict__ prior,
@@ -77,7 +77,7 @@ __global__ __launch_bounds__(256) void sart_update_kernel(DevGeom g, SlotTab S, 
 // terms added in the reference's order from prior[v]); the reference forms
 // each term in double and rounds the sum to float after every term.
 template <int R>
-__global__ __launch_bounds__(256) void huber_prior_kernel(DevGeom g, PriorClass W,
+__global__ __launch_bounds__(64 * CASE_WAVES) void huber_prior_kernel(DevGeom g, PriorClass W,
                                                           float inv_delta,
                                                           const float* __restrict__ x,
                                                           float* __restrict__ prior) {
@@ -103,7 +103,7 @@ __global__ __launch_bounds__(256) void huber_prior_kernel(DevGeom g, PriorClass 
 // x_in and writing x_out keeps the prior's neighbours at their pre-update
 // values, as the separate prior launch does.
 template <bool PRIOR, int R>
-__global__ __launch_bounds__(256) void sart_update_fused_kernel(
+__global__ __launch_bounds__(64 * CASE_WAVES) void sart_update_fused_kernel(
     DevGeom g, SlotTab S, int n_slots, const float* __restrict__ diff,
     const float* __restrict__ x_in, float* __restrict__ x_out, PriorClass W, float inv_delta,
     float lambda, float beta) {
@@ -218,8 +218,8 @@ hipError_t sbp_t(const DevGeom& g, const SlotTab& S, int n, float* img, const vo
                  hipStream_t st) {
     return by_sbp_rows<8>(g, [&](auto rows) {
         constexpr int R = decltype(rows)::value;
-        hipLaunchKernelGGL((sbp_kernel<TP, R>), dim3(volume_tiles(g, R * CASE_WAVES)), dim3(256),
-                           0, st, g, S, n, (const TP*)prj, img);
+        hipLaunchKernelGGL((sbp_kernel<TP, R>), dim3(volume_tiles(g, R * CASE_WAVES)),
+                           dim3(64 * CASE_WAVES), 0, st, g, S, n, (const TP*)prj, img);
         return hipGetLastError();
     });
 }
@@ -315,12 +315,12 @@ hipError_t launch_sart_update(const DevGeom& g, const ViewTab* views, int a0, in
     if (!fill_slots(S, views, a0, a1, g.src_y)) return hipErrorInvalidValue;
     return by_sbp_rows<4>(g, [&](auto rows) {
         constexpr int R = decltype(rows)::value;
-        const dim3 grid(volume_tiles(g, R * CASE_WAVES));
+        const dim3 grid(volume_tiles(g, R * CASE_WAVES)), block(64 * CASE_WAVES);
         if (prior)
-            hipLaunchKernelGGL((sart_update_kernel<float, true, R>), grid, dim3(256), 0, st, g, S,
+            hipLaunchKernelGGL((sart_update_kernel<float, true, R>), grid, block, 0, st, g, S,
                                a1 - a0, diff_rows, img, prior, lambda, beta);
         else
-            hipLaunchKernelGGL((sart_update_kernel<float, false, R>), grid, dim3(256), 0, st, g,
+            hipLaunchKernelGGL((sart_update_kernel<float, false, R>), grid, block, 0, st, g,
                                S, a1 - a0, diff_rows, img, nullptr, lambda, 0.0f);
         return hipGetLastError();
     });
@@ -334,7 +334,7 @@ hipError_t launch_huber_prior(const DevGeom& g, float* prior, const float* img, 
     return by_sbp_rows<4>(g, [&](auto rows) {
         constexpr int R = decltype(rows)::value;
         hipLaunchKernelGGL(huber_prior_kernel<R>, dim3(volume_tiles(g, R * CASE_WAVES)),
-                           dim3(256), 0, st, g, W, 1.0f / delta, img, prior);
+                           dim3(64 * CASE_WAVES), 0, st, g, W, 1.0f / delta, img, prior);
         return hipGetLastError();
     });
 }
@@ -349,12 +349,12 @@ hipError_t launch_sart_update_fused(const DevGeom& g, const ViewTab* views, int 
     const PriorClass W = prior_params(W27, OSTR_PRIOR_HYPERBOLA, delta);
     return by_sbp_rows<4>(g, [&](auto rows) {
         constexpr int R = decltype(rows)::value;
-        const dim3 grid(volume_tiles(g, R * CASE_WAVES));
+        const dim3 grid(volume_tiles(g, R * CASE_WAVES)), block(64 * CASE_WAVES);
         if (beta != 0.0f)
-            hipLaunchKernelGGL((sart_update_fused_kernel<true, R>), grid, dim3(256), 0, st, g, S,
+            hipLaunchKernelGGL((sart_update_fused_kernel<true, R>), grid, block, 0, st, g, S,
                                a1 - a0, diff_rows, x_in, x_out, W, 1.0f / delta, lambda, beta);
         else
-            hipLaunchKernelGGL((sart_update_fused_kernel<false, R>), grid, dim3(256), 0, st, g, S,
+            hipLaunchKernelGGL((sart_update_fused_kernel<false, R>), grid, block, 0, st, g, S,
                                a1 - a0, diff_rows, x_in, x_out, W, 0.0f, lambda, 0.0f);
         return hipGetLastError();
     });

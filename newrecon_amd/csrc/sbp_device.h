@@ -39,7 +39,11 @@ namespace ostr {
 // Tile shape: R voxel rows (y) per wave, NW waves per work-group, 64 voxels
 // along x, one slice. The single-case kernels have CASE_WAVES waves and the
 // rows of by_sbp_rows, the batched kernels take the shape from their caller.
-constexpr int CASE_WAVES = 4;
+// The waves of a group share nothing, and a group's registers are free for the
+// next one only when its last wave ends: with 4, 2 and 1 waves a clinical
+// iteration took 2850 / 2817 / 2794 us, the accelerated one at 200x100x20 38.6 /
+// 37.2 / 37.4, at 256x256x48 173.1 / 174.9 / 172.3.
+constexpr int CASE_WAVES = 1;
 constexpr int TILE_X = 64;
 // prior_rows modes (by_prior_mode)
 constexpr int PRIOR_INTERIOR = 0, PRIOR_EDGE = 1, PRIOR_GENERIC = 2;
@@ -435,7 +439,7 @@ inline unsigned volume_tiles(const DevGeom& g, int tile_y) {
 // geometry, R <= MOST. More rows share a lane's tap columns and the prior's
 // window (about 20 + 9 of the ~330 issue slots per voxel at R = 8), fewer keep
 // more waves in flight. By the waves the volume makes at R = 1; 3 views, FP32,
-// hyperbola, update_fused us at R = 2 / 4 / 8: 8000 waves (200x100x20 voxels)
+// hyperbola, update_fused us (4 waves per group) at R = 2 / 4 / 8: 8000 waves (200x100x20 voxels)
 // 12.9 / 15.8 / 22.6, 16000 19.6 / 19.5 / 24.5, 49152 (256x256x48) 39.7 / 36.2 /
 // 41.4, 150183 (701x333x41) 101 / 85.5 / 86.0, 360000 (1000x500x45) 242 / 200 /
 // 189. The OS-SART updates carry a second sum per row and are faster at R = 4

@@ -10,7 +10,7 @@
 namespace ostr {
 
 template <int POT, typename TI, typename TP, int R>
-__global__ __launch_bounds__(256) void update_fused_kernel(
+__global__ __launch_bounds__(64 * CASE_WAVES) void update_fused_kernel(
     DevGeom g, SlotTab S, int n_slots, const TP* __restrict__ hsub, const TI* __restrict__ x_in,
     TI* __restrict__ x_out, const float* __restrict__ d, PriorClass W, float inv_delta,
     float beta, float capl_scale, int guard) {
@@ -25,7 +25,7 @@ __global__ __launch_bounds__(256) void update_fused_kernel(
 // x_out, the same epilogue (update_rows). h detector-row-major. R rows per
 // lane (matched_row_count).
 template <int POT, typename TI, typename TP, int R>
-__global__ __launch_bounds__(256) void update_fused_matched_kernel(
+__global__ __launch_bounds__(64 * CASE_WAVES) void update_fused_matched_kernel(
     DevGeom g, MatchedSlots S, int n_slots, const TP* __restrict__ hsub,
     const TI* __restrict__ x_in, TI* __restrict__ x_out, const float* __restrict__ d,
     PriorClass W, float inv_delta, float beta, float capl_scale, int guard) {
