@@ -439,11 +439,11 @@ inline unsigned volume_tiles(const DevGeom& g, int tile_y) {
 // geometry, R <= MOST. More rows share a lane's tap columns and the prior's
 // window (about 20 + 9 of the ~330 issue slots per voxel at R = 8), fewer keep
 // more waves in flight. By the waves the volume makes at R = 1; 3 views, FP32,
-// hyperbola, update_fused us (4 waves per group) at R = 2 / 4 / 8: 8000 waves (200x100x20 voxels)
-// 12.9 / 15.8 / 22.6, 16000 19.6 / 19.5 / 24.5, 49152 (256x256x48) 39.7 / 36.2 /
-// 41.4, 150183 (701x333x41) 101 / 85.5 / 86.0, 360000 (1000x500x45) 242 / 200 /
-// 189. The OS-SART updates carry a second sum per row and are faster at R = 4
-// throughout (1000x500x45 182 us against 204 at R = 8): MOST = 4.
+// hyperbola, update_fused us (4 waves per group) at R = 2 / 4 / 8: 8000 waves
+// (200x100x20 voxels) 12.9 / 15.8 / 22.6, 16000 19.6 / 19.5 / 24.5, 49152
+// (256x256x48) 39.7 / 36.2 / 41.4, 150183 (701x333x41) 101 / 85.5 / 86.0, 360000
+// (1000x500x45) 242 / 200 / 189. The OS-SART updates carry a second sum per row and
+// are faster at R = 4 throughout (1000x500x45 182 us against 204 at R = 8): MOST = 4.
 template <int MOST, typename F>
 hipError_t by_sbp_rows(const DevGeom& g, F f) {
     const int64_t waves = (int64_t)((g.nx + TILE_X - 1) / TILE_X) * g.ny * g.nz;
