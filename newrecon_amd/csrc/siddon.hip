@@ -156,18 +156,29 @@ __device__ __forceinline__ void plain_steps(float& xn, float& yn, float& zn, uin
 #undef OSTR_STEP
 }
 
-// A bound T such that from any state with at < T - k inc (and the voxel inside)
-// the next k steps are all taken, inside the volume, inc being the smallest
-// axis increment. A step moves `at` on by at most inc (that axis crosses a
-// plane at least so often), so k steps end before thr. A voxel index is
-// monotonic and can leave the volume only at its exit face's crossing, at or
-// after lmax up to rounding: a crossing is a running sum of at most n
-// increments, each sum off by half an ulp of at most `scale` and the increment
-// by half an ulp of itself, the face's parameter by a few ulps.
-__device__ __forceinline__ float plain_until(float thr, float lmin, float lmax, unsigned n) {
+// Upper end of an axis' plain steps: its exit parameter less the error by which
+// its exit crossing can come early. That crossing is (plane - s) / d, the plane
+// and the difference rounded, plus increments ext / n / d, and hi is (p0 - s) / d
+// + ext / d: each rounding is at most half an ulp of |p0| + |s| + ext over |d|,
+// fewer than 8 of them together, whatever hi itself is. A ray almost parallel to
+// the axis' planes has a large error (7e-3 at 100 mm and d = 1 um); along a
+// parallel one the index never moves.
+__device__ __forceinline__ float plain_exit(const Axis& a, float s, float e, float p0, float ext) {
+    if (s == e) return a.hi;
+    const float reach = fabsf(p0) + fabsf(s) + ext;
+    return fmaf(-0x1p-21f * reach, __builtin_amdgcn_rcpf(fabsf(e - s)), a.hi);
+}
+
+// A bound T such that the voxel is inside and the step is taken from every state
+// whose `at` is below it: below the stop threshold and below every axis' exit
+// crossing. exit: the least plain_exit, in which a crossing still counts as
+// exact but for its running sum of at most n increments, each sum off by half an
+// ulp of at most `scale`.
+__device__ __forceinline__ float plain_until(float thr, float exit, float lmin, float lmax,
+                                             unsigned n) {
     const float scale = fmaxf(fmaxf(1.0f, fabsf(lmin)), fabsf(lmax));
     const float rounding = (float)(n + 16u) * 0x1p-23f * scale;
-    return fminf(thr, lmax) - rounding;
+    return fminf(thr, exit) - rounding;
 }
 
 // One Siddon ray from the source S to the bin centre E. Returns the weighted
@@ -299,10 +310,20 @@ __device__ __forceinline__ float walk(const DevGeom& g, const VolReader<TI>& img
         float segA[WALK_BATCH], vA[WALK_BATCH], segB[WALK_BATCH], vB[WALK_BATCH];
         uint32_t offA[WALK_BATCH], offB[WALK_BATCH];
         bool okA[WALK_BATCH], okB[WALK_BATCH];
+        // `at` is at most the next crossing of the axis with the smallest
+        // increment, which moves on by inc when it is crossed: the k-th state
+        // from the start lies at or before `first` + k inc, and the k-th from a
+        // later one at or before at + (k + 1) inc. (`at` itself may start
+        // before lmin, where an almost parallel axis' first crossing is off.)
         const float inc = fminf(fminf(fabsf(X.inc), fabsf(Y.inc)), fabsf(Z.inc));
-        const float end = plain_until(thr, lmin, lmax, max(nx, max(ny, nz)));
+        const float first = inc == fabsf(X.inc) ? X.next : inc == fabsf(Y.inc) ? Y.next : Z.next;
+        const float exit = fminf(fminf(plain_exit(X, sx, ex, g.x_p0, g.ext_x),
+                                       plain_exit(Y, sy, ey, g.y_p0, g.ext_y)),
+                                 plain_exit(Z, sz, ez, g.z_p0, g.ext_z));
+        const float end = plain_until(thr, exit, lmin, lmax, max(nx, max(ny, nz)));
         const float plain = fmaf(-2.0f * WALK_BATCH, inc, end);  // two batches before it
-        if (at < fmaf(-3.0f * WALK_BATCH, inc, end) && inside()) {
+        // three batches from the start
+        if (first < fmaf(1.0f - 3.0f * WALK_BATCH, inc, end) && inside()) {
             auto steps = [&](float (&seg)[WALK_BATCH], uint32_t (&off)[WALK_BATCH]) {
                 plain_steps(X.next, Y.next, Z.next, px, py, pz, at, cur, X.inc, Y.inc, Z.inc,
                             sxs, sys, szs, len, seg, off);
