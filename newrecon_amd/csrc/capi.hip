@@ -253,6 +253,13 @@ DevGeom make_dev_geom(const ostr_geom& g) {
     d.last_x = std::fma((float)(g.nx - 1), g.dx, g.x_p0);
     d.last_y = std::fma((float)(g.ny - 1), g.dy, g.y_p0);
     d.last_z = std::fma((float)(g.nz - 1), g.dz, g.z_p0);
+    // |source x| and |source z| are at most source_r
+    const auto early = [](float p0, float s, float ext, float h) {
+        return (float)(0x1p-21 * ((double)std::fabs(p0) + std::fabs(s) + ext) / h);
+    };
+    d.early_x = early(g.x_p0, g.source_r, d.ext_x, g.dx);
+    d.early_y = early(g.y_p0, g.source_y, d.ext_y, g.dy);
+    d.early_z = early(g.z_p0, g.source_r, d.ext_z, g.dz);
     return d;
 }
 

@@ -18,6 +18,9 @@ struct DevGeom {
     float top_x, top_y, top_z;   // fma(n, h, p0): upper face of the volume
     float hp_x, hp_y, hp_z;      // h + p0: upper face of voxel 0
     float last_x, last_y, last_z;// fma(n-1, h, p0): lower face of the last voxel
+    // by how many increments a walk's exit crossing may come before the exit
+    // parameter: 2^-21 (|p0| + |s| + ext) / h (plain_exit in siddon.hip)
+    float early_x, early_y, early_z;
 };
 
 // Per-slot view table entry: source x, source z, cos(theta), sin(theta), and

@@ -105,15 +105,13 @@ __device__ __forceinline__ float stop_threshold(float lmax) {
 
 // Upper end of an axis' plain steps: its exit parameter less the error by which
 // its exit crossing can come early. That crossing is (plane - s) / d, the plane
-// and the difference rounded, plus increments ext / n / d, and hi is (p0 - s) / d
-// + ext / d: each rounding is at most half an ulp of |p0| + |s| + ext over |d|,
-// fewer than 8 of them together, whatever hi itself is. A ray almost parallel to
-// the axis' planes has a large error (7e-3 at 100 mm and d = 1 um); along a
-// parallel one the index never moves.
-__device__ __forceinline__ float plain_exit(const Axis& a, float s, float e, float p0, float ext) {
-    if (s == e) return a.hi;
-    const float reach = fabsf(p0) + fabsf(s) + ext;
-    return fmaf(-0x1p-21f * reach, __builtin_amdgcn_rcpf(fabsf(e - s)), a.hi);
+// and the difference rounded, plus increments h / d, and hi is (p0 - s) / d +
+// ext / d: each rounding is at most half an ulp of |p0| + |s| + ext over |d|, fewer
+// than 8 of them together, whatever hi itself is; in increments, DevGeom's k. A
+// ray almost parallel to the axis' planes has a large error (7e-3 at 100 mm and
+// d = 1 um); along a parallel one the index never moves.
+__device__ __forceinline__ float plain_exit(const Axis& a, float s, float e, float k) {
+    return s == e ? a.hi : fmaf(-k, fabsf(a.inc), a.hi);
 }
 
 // A bound T such that the voxel is inside and the step is taken from every state
@@ -264,9 +262,9 @@ __device__ __forceinline__ float walk(const DevGeom& g, const VolReader<TI>& img
         // before lmin, where an almost parallel axis' first crossing is off.)
         const float inc = fminf(fminf(fabsf(X.inc), fabsf(Y.inc)), fabsf(Z.inc));
         const float first = inc == fabsf(X.inc) ? X.next : inc == fabsf(Y.inc) ? Y.next : Z.next;
-        const float exit = fminf(fminf(plain_exit(X, sx, ex, g.x_p0, g.ext_x),
-                                       plain_exit(Y, sy, ey, g.y_p0, g.ext_y)),
-                                 plain_exit(Z, sz, ez, g.z_p0, g.ext_z));
+        const float exit = fminf(fminf(plain_exit(X, sx, ex, g.early_x),
+                                       plain_exit(Y, sy, ey, g.early_y)),
+                                 plain_exit(Z, sz, ez, g.early_z));
         const float end = plain_until(thr, exit, lmin, lmax, max(nx, max(ny, nz)));
         const float plain = fmaf(-2.0f * WALK_BATCH, inc, end);  // two batches before it
         // three batches from the start
