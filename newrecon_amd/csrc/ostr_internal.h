@@ -535,34 +535,47 @@ __device__ __forceinline__ int xcd_tile(int b, int nblocks) {
 // launch walk the same volume rows, so their tiles over one detector row belong
 // on one XCD at one time, where its L2 serves them together. So the tiles are
 // taken in bands: one row of tiles (64 columns x TJ rows each) of all views,
-// view fastest; band b goes to XCD b % 8 (work-group w runs on XCD w % 8). A
+// view fastest; band b goes to XCD b % 8 (work-group w runs on XCD w % 8).
+// Detectors of few bands go column by column instead (ray_by_columns). A
 // 3-view clinical subset fetched 885 MB through the L2s with tiles dealt in
 // blocks of 64 x 64 bins of one view (201 MB of volume, 82 MB of sinograms),
 // 360 MB in bands; fproj_h 180 -> 170 us.
 struct RayTile {
     int slot, ti, tj;
 };
+// Units dealt to the XCDs: whole bands, or, where a detector has too few of them
+// for an even share, (band, tile column) pairs of all views, bands fastest. fproj
+// in bands and in columns, 15 views: 2048x4 bins 29.2 and 10.9 us, 2048x16 36.4
+// and 23.7, 2048x40 61.0 and 42.8, 2048x80 (20 bands) 85.9 and 74.4, 2048x100 89.7
+// and 89.0; 1024x40 34.2 and 26.2; 256x60 14.7 and 15.4, 256x80 19.0 and 17.3,
+// 256x100 19.4 and 19.7, 256x128 23.3 and 24.0.
+__host__ __device__ inline bool ray_by_columns(int tiles_j) { return tiles_j < 24; }
 // Tile of work-group w of a launch of ray_grid() groups; false past the last
-// band.
-__device__ __forceinline__ bool ray_tile(int w, int n_slots, int tiles_i, int tiles_j,
+// unit.
+__host__ __device__ inline bool ray_tile(int w, int n_slots, int tiles_i, int tiles_j,
                                          RayTile& t) {
     const int u = w >> 3, rest = u / n_slots;
     t.slot = u - rest * n_slots;
+    if (ray_by_columns(tiles_j)) {
+        const int unit = rest * 8 + (w & 7);
+        t.ti = unit / tiles_j;
+        t.tj = unit % tiles_j;
+        return t.ti < tiles_i;
+    }
     t.ti = rest % tiles_i;
     t.tj = (rest / tiles_i) * 8 + (w & 7);
     return t.tj < tiles_j;
 }
 inline int64_t ray_grid(int n_slots, int tiles_i, int tiles_j) {
+    if (ray_by_columns(tiles_j)) return ((int64_t)tiles_i * tiles_j + 7) / 8 * 8 * n_slots;
     return (int64_t)n_slots * tiles_i * ((tiles_j + 7) / 8 * 8);
 }
-// The same bands for a launch that hands each XCD one contiguous range of a
+// The same units for a launch that hands each XCD one contiguous range of a
 // case's tile indices (BatchWalk): position t of the n_slots tiles_i tiles_j
-// tiles, whose eighths cover every eighth band (bands 0, 8, 16, ..., 1, 9, 17,
+// tiles, whose eighths cover every eighth unit (units 0, 8, 16, ..., 1, 9, 17,
 // ..., 7, 15, ...).
-__device__ __forceinline__ RayTile ray_tile_of_position(int t, int n_slots, int tiles_i,
-                                                        int tiles_j) {
-    const int per = n_slots * tiles_i, p = t / per, u = t - p * per;
-    const int q = tiles_j / 8, rem = tiles_j % 8;  // class k holds q + (k < rem) bands
+__host__ __device__ inline int ray_unit_of_position(int p, int units) {
+    const int q = units / 8, rem = units % 8;  // class k holds q + (k < rem) units
     int k, m;
     if (p < rem * (q + 1)) {
         k = p / (q + 1);
@@ -572,7 +585,16 @@ __device__ __forceinline__ RayTile ray_tile_of_position(int t, int n_slots, int 
         k = rem + p2 / q;
         m = p2 % q;
     }
-    return RayTile{u % n_slots, u / n_slots, k + 8 * m};
+    return k + 8 * m;
+}
+__host__ __device__ inline RayTile ray_tile_of_position(int t, int n_slots, int tiles_i,
+                                                        int tiles_j) {
+    if (ray_by_columns(tiles_j)) {
+        const int p = t / n_slots, u = ray_unit_of_position(p, tiles_i * tiles_j);
+        return RayTile{t - p * n_slots, u / tiles_j, u % tiles_j};
+    }
+    const int per = n_slots * tiles_i, p = t / per, u = t - p * per;
+    return RayTile{u % n_slots, u / n_slots, ray_unit_of_position(p, tiles_j)};
 }
 
 // Tile walk of a batched launch (one-tile-per-group and persistent grids
