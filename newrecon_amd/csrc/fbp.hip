@@ -21,9 +21,9 @@
 // order out), multiply by the spectrum, run the decimation-in-frequency
 // inverse with conjugate twiddles (bit-reversed order out) and store rows
 // i < nbx from their bit-reversed positions, so no reordering pass is needed.
-// From L = 1024 on fbp_filter_reg_kernel holds 16 points per thread and
-// sequence in registers through up to four radix-2 stages between LDS
-// exchanges; below that fbp_filter_kernel passes over LDS two stages at a time.
+// From L = 1024 on (there with many groups) fbp_filter_reg_kernel holds 16 points
+// per thread and sequence in registers through up to four radix-2 stages between
+// LDS exchanges; otherwise fbp_filter_kernel passes over LDS two stages at a time.
 // Both make the same operations.
 #include <type_traits>
 
@@ -616,12 +616,19 @@ hipError_t launch_fbp_filter(const DevGeom& g, const ViewTab* views, int a0, int
                    : in_registers(logl_c, std::integral_constant<int, 1>());
     };
     switch (logl) {
-        case 10: return by_seq(std::integral_constant<int, 10>());
+        // one wave per 1024 points: faster where the groups are more than two per
+        // CU (9 views of 300x300 bins, 675 groups, 21.4 us in passes and 19.2; 25
+        // of 512x1200, 7500 groups, 128 and 91), slower where a group's latency
+        // is the launch's (one view of 512x222 16.6 and 19.3, 5 of 512x400, 500
+        // groups, 18.9 and 20.5)
+        case 10:
+            if (grid.x > 512) return by_seq(std::integral_constant<int, 10>());
+            break;
         case 11: return by_seq(std::integral_constant<int, 11>());
         case 12: return by_seq(std::integral_constant<int, 12>());
         case 13: return by_seq(std::integral_constant<int, 13>());
     }
-    // fewer than 64 threads of 16 points: passes over LDS
+    // passes over LDS: fewer than 64 threads of 16 points, or few groups
     const hipError_t e = spectrum_by_passes();
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(fbp_filter_kernel<2>, grid, dim3(FFT_THREADS), lds, st, g, views, a0,
