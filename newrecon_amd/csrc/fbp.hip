@@ -156,6 +156,8 @@ __device__ void fft_dif_inverse(float2* buf, int seq, int logl, const float2* tw
 template <int LOGL>
 struct FftPlan {
     static constexpr int T = 1 << (LOGL - 4), PASSES = (LOGL + 3) / 4;
+    // column pairs of a filter group; at 8192 points two would take all 160 KB of LDS
+    static constexpr int SEQ = LOGL < 13 ? 2 : 1;
     static constexpr int stages(int p) { return LOGL - 4 * p < 4 ? LOGL - 4 * p : 4; }
 };
 __device__ __forceinline__ int fft_swz(int i) { return i ^ ((i >> 4) & 31); }
@@ -345,12 +347,12 @@ __device__ __forceinline__ int xcd_contiguous(int b, int n) {
 // Group = SEQ column pairs (2 SEQ columns from j0) of one slot. LDS: L/2 + SEQ L
 // float2. p is [slot][nbx][nby] from slot a0, q the same or, with rows,
 // detector-row-major [slot][nby][nbx]; vec: nby % 4 == 0 and p, q 16-byte
-// aligned (SEQ = 2: float4 row loads and stores).
-template <int SEQ>
+// aligned (float4 row loads and stores).
 __global__ __launch_bounds__(FFT_THREADS) void fbp_filter_kernel(
     DevGeom g, const ViewTab* __restrict__ views, int a0, int n_slots, int n_chunks, int logl,
     const float2* __restrict__ tw_g, const float2* __restrict__ hs, const float* __restrict__ p,
     float* __restrict__ q, int vec, int rows) {
+    constexpr int SEQ = 2;
     extern __shared__ float2 lds[];
     const int L = 1 << logl;
     float2* tw = lds;
@@ -378,7 +380,7 @@ __global__ __launch_bounds__(FFT_THREADS) void fbp_filter_kernel(
             const float ex = (float)((double)g.x_d0 + ((double)i + 0.5) * (double)g.dbx);
             const float dx = ex - v.x0;
             const float* row = p + base + (int64_t)i * nby;
-            if (SEQ == 2 && vec) {
+            if (vec) {
                 const float4 r4 = *(const float4*)row;
                 val[0] = r4.x;
                 val[1] = r4.y;
@@ -426,7 +428,7 @@ __global__ __launch_bounds__(FFT_THREADS) void fbp_filter_kernel(
             val[2 * s + 1] = y.y;
         }
         float* row = q + base + (int64_t)i * nby;
-        if (SEQ == 2 && vec) {
+        if (vec) {
             *(float4*)row = make_float4(val[0], val[1], val[2], val[3]);
         } else {
 #pragma unroll
@@ -443,7 +445,7 @@ __global__ __launch_bounds__(FFT_THREADS) void fbp_filter_kernel(
 // passes over LDS. Bound by VALU issue (two waves per SIMD, 245 VGPRs) and the
 // 16-byte pieces of p. 9 views of 2048x1664 bins:
 // 365 us in passes, 174 here (ROWS 179); 25 of 1106x777 460, 253 (ROWS 210).
-template <int LOGL, int SEQ, bool ROWS>
+template <int LOGL, bool ROWS>
 __global__ __launch_bounds__(FftPlan<LOGL>::T) __attribute__((amdgpu_waves_per_eu(2)))
 void fbp_filter_reg_kernel(
     DevGeom g, const ViewTab* __restrict__ views, int a0, int n_slots, int n_chunks,
@@ -451,6 +453,7 @@ void fbp_filter_reg_kernel(
     float* __restrict__ q, int vec) {
     extern __shared__ float2 lds[];
     constexpr int L = 1 << LOGL, T = FftPlan<LOGL>::T, LAST = FftPlan<LOGL>::PASSES - 1;
+    constexpr int SEQ = FftPlan<LOGL>::SEQ;
     float2* tw = lds;
     float2* buf = lds + L / 2;
     const int t = threadIdx.x;
@@ -574,28 +577,26 @@ hipError_t launch_fbp_filter(const DevGeom& g, const ViewTab* views, int a0, int
     if (n_slots <= 0) return hipSuccess;
     const int logl = fbp_fft_log2(g.nbx);
     const int L = 1 << logl;
+    if (logl > 13) return hipErrorInvalidValue;
     float2* tw = spec;        // L/2
     float2* hs = spec + L / 2;  // L
     const size_t spec_lds = (size_t)(L + L / 2) * sizeof(float2);
-    const size_t lds2 = (size_t)(L / 2 + 2 * L) * sizeof(float2);
-    const size_t lds1 = (size_t)(L / 2 + L) * sizeof(float2);
-    if (lds1 > (size_t)lds_limit || spec_lds > (size_t)lds_limit) return hipErrorInvalidValue;
+    const int seq = logl < 13 ? 2 : 1;  // column pairs per group (FftPlan::SEQ)
+    const size_t lds = (size_t)(L / 2 + seq * L) * sizeof(float2);
+    if (lds > (size_t)lds_limit || spec_lds > (size_t)lds_limit) return hipErrorInvalidValue;
     const int vec = (g.nby % 4 == 0) && ((uintptr_t)p % 16 == 0) && ((uintptr_t)q % 16 == 0);
-    // two column pairs per group where they fit (at 8192 points in registers one)
-    const bool two = lds2 <= (size_t)lds_limit && logl < 13;
-    const int n_chunks = two ? (g.nby + 3) / 4 : (g.nby + 1) / 2;
+    const int n_chunks = (g.nby + 2 * seq - 1) / (2 * seq);
     const dim3 grid((unsigned)(n_chunks * n_slots));
-    const size_t lds = two ? lds2 : lds1;
     // at most 1024 points; 256 threads, which one wave of 16 points each is slower than
     auto spectrum_by_passes = [&] {
         hipLaunchKernelGGL(fbp_spectrum_kernel, dim3(1), dim3(FFT_THREADS), spec_lds, st, taps,
                            ntaps, g.nbx, logl, tw, hs);
         return hipGetLastError();
     };
-    auto in_registers = [&](auto logl_c, auto seq_c) {
-        constexpr int LOGL = decltype(logl_c)::value, SEQ = decltype(seq_c)::value;
-        const auto kernel = rows ? fbp_filter_reg_kernel<LOGL, SEQ, true>
-                                 : fbp_filter_reg_kernel<LOGL, SEQ, false>;
+    auto in_registers = [&](auto logl_c) {
+        constexpr int LOGL = decltype(logl_c)::value;
+        const auto kernel = rows ? fbp_filter_reg_kernel<LOGL, true>
+                                 : fbp_filter_reg_kernel<LOGL, false>;
         hipError_t err = allow_lds((const void*)kernel, lds);
         if (err != hipSuccess) return err;
         if constexpr (LOGL > 10) {
@@ -608,12 +609,8 @@ hipError_t launch_fbp_filter(const DevGeom& g, const ViewTab* views, int a0, int
             return err;
         }
         hipLaunchKernelGGL(kernel, grid, dim3(FftPlan<LOGL>::T), lds, st, g, views, a0, n_slots,
-                           n_chunks, tw, hs, p, q, SEQ == 2 ? vec : 0);
+                           n_chunks, tw, hs, p, q, vec);
         return hipGetLastError();
-    };
-    auto by_seq = [&](auto logl_c) {
-        return two ? in_registers(logl_c, std::integral_constant<int, 2>())
-                   : in_registers(logl_c, std::integral_constant<int, 1>());
     };
     switch (logl) {
         // one wave per 1024 points: faster where the groups are more than two per
@@ -622,16 +619,16 @@ hipError_t launch_fbp_filter(const DevGeom& g, const ViewTab* views, int a0, int
         // is the launch's (one view of 512x222 16.6 and 19.3, 5 of 512x400, 500
         // groups, 18.9 and 20.5)
         case 10:
-            if (grid.x > 512) return by_seq(std::integral_constant<int, 10>());
+            if (grid.x > 512) return in_registers(std::integral_constant<int, 10>());
             break;
-        case 11: return by_seq(std::integral_constant<int, 11>());
-        case 12: return by_seq(std::integral_constant<int, 12>());
-        case 13: return by_seq(std::integral_constant<int, 13>());
+        case 11: return in_registers(std::integral_constant<int, 11>());
+        case 12: return in_registers(std::integral_constant<int, 12>());
+        case 13: return in_registers(std::integral_constant<int, 13>());
     }
     // passes over LDS: fewer than 64 threads of 16 points, or few groups
     const hipError_t e = spectrum_by_passes();
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(fbp_filter_kernel<2>, grid, dim3(FFT_THREADS), lds, st, g, views, a0,
+    hipLaunchKernelGGL(fbp_filter_kernel, grid, dim3(FFT_THREADS), lds, st, g, views, a0,
                        n_slots, n_chunks, logl, tw, hs, p, q, vec, rows);
     return hipGetLastError();
 }
