@@ -216,7 +216,7 @@ bool fill_slots(SlotTab& S, const ViewTab* host_views, int a0, int a1, float src
 template <typename TP>
 hipError_t sbp_t(const DevGeom& g, const SlotTab& S, int n, float* img, const void* prj,
                  hipStream_t st) {
-    return by_sbp_rows<8>(g, [&](auto rows) {
+    return by_sbp_rows<8>(g, SBP_ROWS_LINE, [&](auto rows) {
         constexpr int R = decltype(rows)::value;
         hipLaunchKernelGGL((sbp_kernel<TP, R>), dim3(volume_tiles(g, R * CASE_WAVES)),
                            dim3(64 * CASE_WAVES), 0, st, g, S, n, (const TP*)prj, img);
@@ -308,12 +308,15 @@ hipError_t launch_transpose_bins(const void* src, void* dst, int n_slots, int nb
 
 // `views` is the HOST copy of the slot table (slot parameters go to the kernel
 // by value). prj is detector-row-major [slot][nby][nbx].
+// The OS-SART updates carry a second sum per row and are faster at 4 rows than at
+// 8 throughout (1000x500x45 voxels, 3 views, with the prior 179 and 204 us, without
+// 86 and 88; 1400x600x60 389 and 423).
 hipError_t launch_sart_update(const DevGeom& g, const ViewTab* views, int a0, int a1,
                               float* img, const float* diff_rows, const float* prior,
                               float lambda, float beta, hipStream_t st) {
     SlotTab S;
     if (!fill_slots(S, views, a0, a1, g.src_y)) return hipErrorInvalidValue;
-    return by_sbp_rows<4>(g, [&](auto rows) {
+    return by_sbp_rows<4>(g, SBP_ROWS_LINE, [&](auto rows) {
         constexpr int R = decltype(rows)::value;
         const dim3 grid(volume_tiles(g, R * CASE_WAVES)), block(64 * CASE_WAVES);
         if (prior)
@@ -326,12 +329,13 @@ hipError_t launch_sart_update(const DevGeom& g, const ViewTab* views, int a0, in
     });
 }
 
+// 1400x600x60 voxels: 226 us at 8 rows per wave, 238 at 4 (256x256x48: 19.4 and 19.0)
 hipError_t launch_huber_prior(const DevGeom& g, float* prior, const float* img, float delta,
                               hipStream_t st) {
     PriorW W27;
     prior_weights(W27.w, 1.0f);
     const PriorClass W = prior_params(W27, OSTR_PRIOR_HYPERBOLA, delta);
-    return by_sbp_rows<4>(g, [&](auto rows) {
+    return by_sbp_rows<8>(g, SBP_ROWS_LINE, [&](auto rows) {
         constexpr int R = decltype(rows)::value;
         hipLaunchKernelGGL(huber_prior_kernel<R>, dim3(volume_tiles(g, R * CASE_WAVES)),
                            dim3(64 * CASE_WAVES), 0, st, g, W, 1.0f / delta, img, prior);
@@ -347,7 +351,7 @@ hipError_t launch_sart_update_fused(const DevGeom& g, const ViewTab* views, int 
     PriorW W27;
     prior_weights(W27.w, 1.0f);
     const PriorClass W = prior_params(W27, OSTR_PRIOR_HYPERBOLA, delta);
-    return by_sbp_rows<4>(g, [&](auto rows) {
+    return by_sbp_rows<4>(g, SBP_ROWS_LINE, [&](auto rows) {
         constexpr int R = decltype(rows)::value;
         const dim3 grid(volume_tiles(g, R * CASE_WAVES)), block(64 * CASE_WAVES);
         if (beta != 0.0f)

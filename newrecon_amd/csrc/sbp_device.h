@@ -438,17 +438,21 @@ inline unsigned volume_tiles(const DevGeom& g, int tile_y) {
 // f(std::integral_constant<int, R>) with R voxel rows per wave for the
 // geometry, R <= MOST. More rows share a lane's tap columns and the prior's
 // window (about 20 + 9 of the ~330 issue slots per voxel at R = 8), fewer keep
-// more waves in flight. By the waves the volume makes at R = 1; 3 views, FP32,
-// hyperbola, update_fused us (4 waves per group) at R = 2 / 4 / 8: 8000 waves
-// (200x100x20 voxels) 12.9 / 15.8 / 22.6, 16000 19.6 / 19.5 / 24.5, 49152
-// (256x256x48) 39.7 / 36.2 / 41.4, 150183 (701x333x41) 101 / 85.5 / 86.0, 360000
-// (1000x500x45) 242 / 200 / 189. The OS-SART updates carry a second sum per row and
-// are faster at R = 4 throughout (1000x500x45 182 us against 204 at R = 8): MOST = 4.
+// more waves in flight. By the waves the volume makes at R = 1: 2 rows below
+// 16000, 8 from `line` on. update_fused of 3 views, FP32, hyperbola, us at R = 2 /
+// 4 / 8: 1920 waves (120x60x16 voxels) 9.8 / 9.2 / 12.2, 8000 (200x100x20) 11.7 /
+// 12.2 / 17.4, 12000 (200x150x20) 15.5 / 13.9 / 19.4, 24576 (256x256x24) 21.4 /
+// 20.6 / 23.4, 49152 (256x256x48) 39.0 / 36.3 / 41.0, 99000 (600x300x33) 66.9 /
+// 58.7 / 58.8, 150183 (701x333x41) 97.8 / 82.7 / 81.9, 208000 (800x400x40) 133 /
+// 114 / 112, 360000 (1000x500x45) 235 / 194 / 186. Around 16000 more views favour
+// fewer rows: 25 views and q2 at 12000 40.2 / 44.1 / 65.9 (the backprojection alone
+// 35.7 / 39.6 / 58.6), at 16000 51.0 / 51.1 / 73.3.
+constexpr int SBP_ROWS_LINE = 200000;
 template <int MOST, typename F>
-hipError_t by_sbp_rows(const DevGeom& g, F f) {
+hipError_t by_sbp_rows(const DevGeom& g, int64_t line, F f) {
     const int64_t waves = (int64_t)((g.nx + TILE_X - 1) / TILE_X) * g.ny * g.nz;
     if (waves < 16000) return f(std::integral_constant<int, 2>());
-    if (MOST < 8 || waves < 200000) return f(std::integral_constant<int, 4>());
+    if (MOST < 8 || waves < line) return f(std::integral_constant<int, 4>());
     return f(std::integral_constant<int, MOST>());
 }
 

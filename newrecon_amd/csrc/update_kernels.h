@@ -64,11 +64,15 @@ hipError_t by_update_types(int potential, int prj_dtype, F f) {
     return hipErrorInvalidValue;
 }
 
+// 8 rows per wave from 120000 waves on for up to 3 views, where the window's loads
+// weigh more: at 701x333x41 voxels (150183 waves) 4 and 8 rows take, us, one view
+// and q2 47.3 and 44.8, Lange with BF16 h 71.7 and 69.7, hyperbola 66.9 and 67.8,
+// but 9 views and q2 111.5 and 116.1.
 template <typename TI>
 hipError_t update_fused_image(const SlotTab& S, const UpdateCall& u, hipStream_t st) {
     return by_update_types(u.potential, u.prj_dtype, [&](auto pot, auto* h) {
         using TP = std::remove_pointer_t<decltype(h)>;
-        return by_sbp_rows<8>(u.g, [&](auto rows) {
+        return by_sbp_rows<8>(u.g, u.n_slots <= 3 ? 120000 : SBP_ROWS_LINE, [&](auto rows) {
             constexpr int R = decltype(rows)::value;
             hipLaunchKernelGGL((update_fused_kernel<decltype(pot)::value, TI, TP, R>),
                                dim3(volume_tiles(u.g, R * CASE_WAVES)), dim3(64 * CASE_WAVES), 0,
