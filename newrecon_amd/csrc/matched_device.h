@@ -83,13 +83,15 @@ inline MatchedSlots matched_slots(const DevGeom& g, const ViewTab* v, int n) {
 
 // Voxel rows per wave, R. More rows share a lane's clipped columns (about 35 of
 // the ~80 instructions per voxel and view at R = 1), fewer keep more waves in
-// flight: R = 4 as long as that leaves the chip's 1024 SIMDs 4 waves each.
-// Accelerated iteration, us: 256x256x48 voxels, 15 views (49152 waves at R = 1)
-// 234 / 186 / 180 at R = 1 / 2 / 4; 200x100x20, 9 views (8000 waves) 42 / 40 /
-// 46.
+// flight. Fused update of 9 views, us at R = 1 / 2 / 4 by the waves at R = 1: 1920
+// (120x60x16 voxels) 11.4 / 12.4 / 16.9, 8000 (200x100x20) 23.8 / 19.7 / 20.5, 12000
+// (200x150x20) 31.6 / 26.8 / 25.0, 16000 (200x100x40) 39.8 / 31.4 / 29.8, 24576
+// (256x256x24) 58.3 / 48.7 / 50.1, 49152 (256x256x48) 111 / 90.1 / 88.4, 792000
+// (1400x600x60) 1935 / 1598 / 1587; the transpose alone at 12000 25.6 / 22.1 / 20.7,
+// at 24576 45.7 / 35.6 / 31.5.
 inline int matched_row_count(const DevGeom& g) {
     const int64_t waves = (int64_t)((g.nx + 63) / 64) * g.ny * g.nz;  // at R = 1
-    return waves >= 16384 ? 4 : waves >= 4096 ? 2 : 1;
+    return waves >= 10000 ? 4 : waves >= 4096 ? 2 : 1;
 }
 // f(std::integral_constant<int, R>) for the geometry's row count.
 template <typename F>
