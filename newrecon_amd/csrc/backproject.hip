@@ -48,8 +48,8 @@ __global__ __launch_bounds__(64 * CASE_WAVES) void sart_update_kernel(DevGeom g,
                                                           float* __restrict__ img,
                                                           const float* __restrict__ prior,
                                                           float lambda, float beta) {
-    const TileCoord c = tile_coord<R, CASE_WAVES>(g, xcd_tile(blockIdx.x, gridDim.x));
-    if (c.iy0 >= g.ny) return;  // see sbp_kernel
+    const TileCoord c = tile_coord<R, CASE_WAVES>(g, group_tile());
+    if (c.iy0 >= g.ny || c.iz >= g.nz) return;  // see sbp_kernel
     const VolReader<TP> P(diff, (uint32_t)n_slots * g.nbx * g.nby);
     float total[R], sens[R];
     sbp_rows<TP, R, true>(g, S, n_slots, P, c.ix, c.iy0, c.iz, total, sens);
@@ -107,8 +107,8 @@ __global__ __launch_bounds__(64 * CASE_WAVES) void sart_update_fused_kernel(
     DevGeom g, SlotTab S, int n_slots, const float* __restrict__ diff,
     const float* __restrict__ x_in, float* __restrict__ x_out, PriorClass W, float inv_delta,
     float lambda, float beta) {
-    const TileCoord c = tile_coord<R, CASE_WAVES>(g, xcd_tile(blockIdx.x, gridDim.x));
-    if (c.iy0 >= g.ny) return;  // see sbp_kernel
+    const TileCoord c = tile_coord<R, CASE_WAVES>(g, group_tile());
+    if (c.iy0 >= g.ny || c.iz >= g.nz) return;  // see sbp_kernel
     const uint32_t nvox = (uint32_t)g.nx * g.ny * g.nz;
     const VolReader<float> P(diff, (uint32_t)n_slots * g.nbx * g.nby);
     const VolReader<float> X(x_in, nvox);
@@ -318,7 +318,8 @@ hipError_t launch_sart_update(const DevGeom& g, const ViewTab* views, int a0, in
     if (!fill_slots(S, views, a0, a1, g.src_y)) return hipErrorInvalidValue;
     return by_sbp_rows<4>(g, SBP_ROWS_LINE, [&](auto rows) {
         constexpr int R = decltype(rows)::value;
-        const dim3 grid(volume_tiles(g, R * CASE_WAVES)), block(64 * CASE_WAVES);
+        const dim3 grid = group_grid(volume_tiles(g, R * CASE_WAVES), 64 * CASE_WAVES);
+        const dim3 block(64 * CASE_WAVES);
         if (prior)
             hipLaunchKernelGGL((sart_update_kernel<float, true, R>), grid, block, 0, st, g, S,
                                a1 - a0, diff_rows, img, prior, lambda, beta);
@@ -353,7 +354,8 @@ hipError_t launch_sart_update_fused(const DevGeom& g, const ViewTab* views, int 
     const PriorClass W = prior_params(W27, OSTR_PRIOR_HYPERBOLA, delta);
     return by_sbp_rows<4>(g, SBP_ROWS_LINE, [&](auto rows) {
         constexpr int R = decltype(rows)::value;
-        const dim3 grid(volume_tiles(g, R * CASE_WAVES)), block(64 * CASE_WAVES);
+        const dim3 grid = group_grid(volume_tiles(g, R * CASE_WAVES), 64 * CASE_WAVES);
+        const dim3 block(64 * CASE_WAVES);
         if (beta != 0.0f)
             hipLaunchKernelGGL((sart_update_fused_kernel<true, R>), grid, block, 0, st, g, S,
                                a1 - a0, diff_rows, x_in, x_out, W, 1.0f / delta, lambda, beta);

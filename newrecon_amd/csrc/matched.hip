@@ -20,11 +20,11 @@ __global__ __launch_bounds__(256) void matched_kernel(DevGeom g, MatchedSlots S,
                                                       const TP* __restrict__ prj,
                                                       float* __restrict__ img) {
     const int tiles_x = (g.nx + 63) / 64, tiles_y = (g.ny + 4 * R - 1) / (4 * R);
-    const int t = xcd_tile(blockIdx.x, gridDim.x);
+    const int t = group_tile();
     const int ix = (t % tiles_x) * 64 + (threadIdx.x & 63);
     const int iy0 = ((t / tiles_x) % tiles_y) * 4 * R + (threadIdx.x >> 6) * R;
     const int iz = t / tiles_x / tiles_y;
-    if (iy0 >= g.ny) return;
+    if (iy0 >= g.ny || iz >= g.nz) return;
     const VolReader<TP> P(prj, (uint32_t)n_slots * g.nbx * g.nby);
     float total[R];
     matched_rows<TP, R>(g, S, n_slots, cos_weight, P, ix, iy0, iz, total);
@@ -42,10 +42,9 @@ hipError_t matched_t(const DevGeom& g, const MatchedSlots& S, int n, int cos_wei
                      const void* prj, float* img, hipStream_t st) {
     return by_matched_rows(g, [&](auto rows) {
         constexpr int R = decltype(rows)::value;
-        const unsigned grid =
-            (unsigned)((g.nx + 63) / 64) * ((g.ny + 4 * R - 1) / (4 * R)) * g.nz;
-        hipLaunchKernelGGL((matched_kernel<TP, R>), dim3(grid), dim3(256), 0, st, g, S, n,
-                           cos_weight, (const TP*)prj, img);
+        const int64_t tiles = (int64_t)((g.nx + 63) / 64) * ((g.ny + 4 * R - 1) / (4 * R)) * g.nz;
+        hipLaunchKernelGGL((matched_kernel<TP, R>), group_grid(tiles, 256), dim3(256), 0, st, g, S,
+                           n, cos_weight, (const TP*)prj, img);
         return hipGetLastError();
     });
 }

@@ -529,6 +529,18 @@ __device__ __forceinline__ int xcd_tile(int b, int nblocks) {
     return t;
 }
 
+// Grid of one work-group of `threads` per tile. A launch takes fewer than 2^32
+// threads along x: more tiles (volumes of 1 to 3 voxels in x and 2^28 rows) go on
+// along y, the last row of groups past the last tile.
+inline dim3 group_grid(int64_t tiles, int threads) {
+    const int64_t most = ((int64_t)1 << 31) / threads;
+    return tiles <= most ? dim3((unsigned)tiles)
+                         : dim3((unsigned)most, (unsigned)((tiles + most - 1) / most));
+}
+__device__ __forceinline__ int group_tile() {
+    return (int)(blockIdx.y * gridDim.x) + xcd_tile(blockIdx.x, gridDim.x);
+}
+
 // Work-group to tile mapping of the ray kernels. Of a detector's ray tiles
 // only those in the volume's shadow walk (about 15% of the bins at the clinical
 // size), so the XCDs need an even share of the shadow; and the views of a

@@ -29,8 +29,8 @@ __global__ __launch_bounds__(64 * CASE_WAVES) void update_fused_matched_kernel(
     DevGeom g, MatchedSlots S, int n_slots, const TP* __restrict__ hsub,
     const TI* __restrict__ x_in, TI* __restrict__ x_out, const float* __restrict__ d,
     PriorClass W, float inv_delta, float beta, float capl_scale, int guard) {
-    const TileCoord c = tile_coord<R, CASE_WAVES>(g, xcd_tile(blockIdx.x, gridDim.x));
-    if (c.iy0 >= g.ny) return;  // see sbp_kernel
+    const TileCoord c = tile_coord<R, CASE_WAVES>(g, group_tile());
+    if (c.iy0 >= g.ny || c.iz >= g.nz) return;  // see sbp_kernel
     const uint32_t nvox = (uint32_t)g.nx * g.ny * g.nz;
     const VolReader<TP> P(hsub, (uint32_t)n_slots * g.nbx * g.nby);
     const VolReader<TI> X(x_in, nvox);
@@ -91,8 +91,9 @@ hipError_t update_matched_image(const MatchedSlots& S, const UpdateCall& u, hipS
         return by_matched_rows(u.g, [&](auto rows) {
             constexpr int R = decltype(rows)::value;
             hipLaunchKernelGGL((update_fused_matched_kernel<decltype(pot)::value, TI, TP, R>),
-                               dim3(volume_tiles(u.g, R * CASE_WAVES)), dim3(64 * CASE_WAVES), 0,
-                               st, u.g, S, u.n_slots, (const TP*)u.hsub, (const TI*)u.x_in,
+                               group_grid(volume_tiles(u.g, R * CASE_WAVES), 64 * CASE_WAVES),
+                               dim3(64 * CASE_WAVES), 0, st, u.g, S, u.n_slots,
+                               (const TP*)u.hsub, (const TI*)u.x_in,
                                (TI*)u.x_out, u.d, u.W, u.inv_delta, u.beta, u.capl_scale,
                                u.guard);
             return hipGetLastError();
