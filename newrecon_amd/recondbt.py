@@ -19,7 +19,10 @@ from .geometry import Geometry
 from .ostr import DBTSystem
 
 
-# sinogram bytes of one launch over several views
+# Sinogram bytes of one launch over several views (at least one view). ml_dbt holds
+# four sinograms of that size, so up to 4 GiB where view by view it held four
+# views: at 1400x600x60 voxels and 15 views of 2048x1664 bins (204 MB) 818 MB against
+# 55, and 6.6 ms per iteration against 11.6 (6.9 with 128 MiB, 9.0 with 32).
 CHUNK_BYTES = 1 << 30
 
 
@@ -66,7 +69,9 @@ def sart_dbt(geom: Geometry, angles, proj, x0, niter: int, stepsize: float,
 
 def ml_dbt(geom: Geometry, angles, counts, x0, I0, niter: int, stepsize: float,
            saveiter: bool = False, device=None):
-    """ML_dbt.m:61-113. counts: measured counts; I0: a scalar or [V][nbx][nby]."""
+    """ML_dbt.m:61-113. counts: measured counts; I0: a scalar or [V][nbx][nby].
+    Besides counts and images it holds four sinograms of at most CHUNK_BYTES each
+    (set it lower where memory is short)."""
     S = _system(geom, angles, device)
     dev, nv = S.device, S.n_views
     c = _f32(counts, dev)
