@@ -518,8 +518,8 @@ class DBTSystem:
         """Cosine-weighted views filtered along detector x with odd-length taps;
         rows: q detector-row-major [S][nby][nbx]."""
         if q is None:
-            q = torch.empty((a1 - a0, self.geom.nby, self.geom.nbx), device=self.device) \
-                if rows else self.sinogram(a1 - a0)
+            q = torch.empty((a1 - a0, self.geom.nby, self.geom.nbx), dtype=torch.float32,
+                            device=self.device) if rows else self.sinogram(a1 - a0)
         for t, what in ((p, "p"), (taps, "taps"), (q, "q")):
             _f32(t, what)
         if taps.numel() % 2 == 0:
