@@ -91,7 +91,7 @@ class BatchOSTR:
 
     All cases must be fused, on one device, with float32 images and one
     sinogram dtype and prior potential. `tile`: a TileCfg, a dict, or None
-    for the single-case shapes.
+    for DEFAULT_TILE.
     """
 
     def __init__(self, cases: Sequence[OSTR], tile=None):

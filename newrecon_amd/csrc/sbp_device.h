@@ -20,7 +20,8 @@
 // only on (x, slice, view) and the tap row (jlb, fracJ) only on (y, slice,
 // view): a lane computes its column terms once per view and reuses them for
 // the ROWS rows it owns, and the row terms are wave-uniform. Work-group tiles
-// (64 x 32 voxels of one slice) are dealt to XCDs in contiguous ranges.
+// (64 x ROWS NW voxels of one slice, NW waves) are dealt to XCDs in contiguous
+// ranges.
 //
 // The fused update computes, per voxel and in one pass,
 //   capL = M * SBP(h)                      (Tomo_OSTR_gold.cpp:759-771)
