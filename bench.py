@@ -192,8 +192,10 @@ def bench_batch(args, dev):
     torch.cuda.synchronize()
     s_step = (time.perf_counter() - t0) / args.steps
 
-    # kernel durations (events on the launch stream)
+    # kernel durations (events on the launch stream), after an untimed call (a
+    # kernel's first launch loads its code)
     def timed(fn, n=5):
+        fn()
         e = [(torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True))
              for _ in range(n)]
         for a, z in e:
