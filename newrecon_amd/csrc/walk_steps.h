@@ -20,9 +20,10 @@ constexpr int WALK_BATCH = 4;  // walk steps per batch (two batches' gathers in 
 // read-write operands are early-clobber: the first step writes them, the later
 // ones still read the inputs.
 // What bounds the walk now is its gathers, not VALU issue: a wave's lanes stand
-// in up to three slices and two rows, so a gather is ~29 L1 accesses and the
-// texture units are busy 85% of the time (VALU issue 71%). A 3-view clinical
-// subset (fproj_h) took 189 us with flagged batches only, 180 with this.
+// in up to three slices and two rows, so a gather is 26-29 L1 accesses, and the
+// L1 makes one per cycle and CU (texture data units busy 86% of the time, VALU
+// issue 75%). A 3-view clinical subset (fproj_h) took 189 us with flagged batches
+// only, 180 with this.
 __device__ __forceinline__ void plain_steps(float& xn, float& yn, float& zn, uint32_t& px,
                                             uint32_t& py, uint32_t& pz, float& at, float& cur,
                                             float xi, float yi, float zi, uint32_t xs,
