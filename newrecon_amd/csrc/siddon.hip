@@ -131,8 +131,9 @@ __device__ __forceinline__ float plain_until(float thr, float exit, float lmin, 
 // COUNT: also counts in-volume segments of positive length into *nseg.
 // NORM: also accumulates the plain row sum into *norm (sum_norm of the SART
 // walker, Tomo_OSTR.cu:534-539, 601-605: the same segments, added in order,
-// so it equals the ONES walk bit for bit).
-template <bool ONES, bool COUNT, typename TI, bool NORM = false>
+// so it equals the ONES walk bit for bit). HIT: only whether and how long, no
+// steps (the compiler cannot leave out those of plain_steps).
+template <bool ONES, bool COUNT, typename TI, bool NORM = false, bool HIT = false>
 __device__ __forceinline__ float walk(const DevGeom& g, const VolReader<TI>& img, float sx,
                                       float sy, float sz, float ex, float ey, float ez,
                                       bool& hit, float& len_out, int& nseg,
@@ -153,6 +154,10 @@ __device__ __forceinline__ float walk(const DevGeom& g, const VolReader<TI>& img
     if (lmin < Y.lo) lmin = Y.lo;
     if (lmin < Z.lo) lmin = Z.lo;
     if (!(lmin < lmax)) return 0.0f;
+    if (HIT) {
+        hit = true;
+        return 0.0f;
+    }
     axis_entry(X, lmin, sx, ex, g.x_p0, g.dx, g.nx, g.hp_x, g.last_x);
     axis_entry(Y, lmin, sy, ey, g.y_p0, g.dy, g.ny, g.hp_y, g.last_y);
     axis_entry(Z, lmin, sz, ez, g.z_p0, g.dz, g.nz, g.hp_z, g.last_z);
@@ -379,7 +384,8 @@ __device__ __forceinline__ void project_bin(const DevGeom& g, const ViewTab& v, 
         else if (KIND == 2 || KIND == 5)
             s = walk<true, false, TI>(g, vol, v.x0, g.src_y, v.z0, ex, ey, ez, hit, len, nseg);
         else {
-            walk<true, false, TI>(g, vol, v.x0, g.src_y, v.z0, ex, ey, ez, hit, len, nseg);
+            walk<true, false, TI, false, true>(g, vol, v.x0, g.src_y, v.z0, ex, ey, ez, hit, len,
+                                               nseg);
             s = len;
         }
     }
