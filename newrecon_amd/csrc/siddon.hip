@@ -266,14 +266,26 @@ __device__ __forceinline__ float walk(const DevGeom& g, const VolReader<TI>& img
         // later one at or before at + (k + 1) inc. (`at` itself may start
         // before lmin, where an almost parallel axis' first crossing is off.)
         const float inc = fminf(fminf(fabsf(X.inc), fabsf(Y.inc)), fabsf(Z.inc));
-        const float first = inc == fabsf(X.inc) ? X.next : inc == fabsf(Y.inc) ? Y.next : Z.next;
-        const float exit = fminf(fminf(plain_exit(X, sx, ex, g.early_x),
-                                       plain_exit(Y, sy, ey, g.early_y)),
-                                 plain_exit(Z, sz, ez, g.early_z));
-        const float end = plain_until(thr, exit, lmin, lmax, max(nx, max(ny, nz)));
-        const float plain = fmaf(-2.0f * WALK_BATCH, inc, end);  // two batches before it
-        // three batches from the start
-        if (first < fmaf(1.0f - 3.0f * WALK_BATCH, inc, end) && inside()) {
+        // Room for three batches before the stop threshold decides first: a short
+        // walk (a volume of few slices) does without the bound. at is no later
+        // than `first` and `end` is below thr, so the full test, which follows,
+        // would fail as well. fproj_h of 3 views, 1000x500x1 voxels, 1536x1024 bins:
+        // 36.2 -> 35.2 us, fproj_4r 119 -> 115; 1400x600x60 voxels, 2048x1664 bins:
+        // fproj_h 246-248 us both.
+        bool plain_run = at < fmaf(1.0f - 3.0f * WALK_BATCH, inc, thr);
+        float plain = 0.0f;
+        if (plain_run) {
+            const float first =
+                inc == fabsf(X.inc) ? X.next : inc == fabsf(Y.inc) ? Y.next : Z.next;
+            const float exit = fminf(fminf(plain_exit(X, sx, ex, g.early_x),
+                                           plain_exit(Y, sy, ey, g.early_y)),
+                                     plain_exit(Z, sz, ez, g.early_z));
+            const float end = plain_until(thr, exit, lmin, lmax, max(nx, max(ny, nz)));
+            plain = fmaf(-2.0f * WALK_BATCH, inc, end);  // two batches before it
+            // three batches from the start
+            plain_run = first < fmaf(1.0f - 3.0f * WALK_BATCH, inc, end) && inside();
+        }
+        if (plain_run) {
             auto steps = [&](float (&seg)[WALK_BATCH], uint32_t (&off)[WALK_BATCH]) {
                 plain_steps(X.next, Y.next, Z.next, px, py, pz, at, cur, X.inc, Y.inc, Z.inc,
                             sxs, sys, szs, len, seg, off);
