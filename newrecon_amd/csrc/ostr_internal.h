@@ -562,10 +562,33 @@ struct RayTile {
 // and 89.0; 1024x40 34.2 and 26.2; 256x60 14.7 and 15.4, 256x80 19.0 and 17.3,
 // 256x100 19.4 and 19.7, 256x128 23.3 and 24.0.
 __host__ __device__ inline bool ray_by_columns(int tiles_j) { return tiles_j < 24; }
+// Kernels that write (or read) the reference layout, y fastest, and walk volumes of
+// few slices: units of two bands of one tile column, pairs of bands fastest. The
+// walks are short there and the scattered stores are most of the work: in bands the
+// shadow's walks all come first and the stores of the rest after them; down a column
+// both run side by side. fproj in bands and in pairs: 3 views, 1536x1024 bins,
+// 1000x500x1 voxels 37.6 and 35.1 us, 1000x500x16 59.8 and 56.4; 25 views, 1024x800
+// bins, 800x400x12 177 and 165 (precompute_d 304 and 274); 15 views, 2500x130 bins,
+// 2000x100x2 49.3 and 44.8. With more slices the bands' locality counts again: 9
+// views, 640x512 bins, 512x400x30 61.8 and 63.0. The line of tiles: up to about 2560
+// most of a launch is in flight at once, and the XCDs' shares count for more than
+// the order (2 views, 640x512 bins, 512x400x8, 2560 tiles: 13.1 and 14.6).
+__host__ __device__ inline bool ray_by_pairs(int nz, int n_slots, int tiles_i, int tiles_j) {
+    return nz <= 16 && !ray_by_columns(tiles_j) &&
+           (int64_t)n_slots * tiles_i * tiles_j > 2560;
+}
 // Tile of work-group w of a launch of ray_grid() groups; false past the last
-// unit.
+// unit. pairs: by ray_by_pairs, the same for both.
 __host__ __device__ inline bool ray_tile(int w, int n_slots, int tiles_i, int tiles_j,
-                                         RayTile& t) {
+                                         RayTile& t, bool pairs = false) {
+    if (pairs) {
+        const int pairs_j = (tiles_j + 1) >> 1, v = w >> 4, rest = v / n_slots;
+        const int unit = rest * 8 + (w & 7);
+        t.slot = v - rest * n_slots;
+        t.ti = unit / pairs_j;
+        t.tj = 2 * (unit - t.ti * pairs_j) + ((w >> 3) & 1);
+        return t.ti < tiles_i && t.tj < tiles_j;
+    }
     const int u = w >> 3, rest = u / n_slots;
     t.slot = u - rest * n_slots;
     if (ray_by_columns(tiles_j)) {
@@ -578,7 +601,8 @@ __host__ __device__ inline bool ray_tile(int w, int n_slots, int tiles_i, int ti
     t.tj = (rest / tiles_i) * 8 + (w & 7);
     return t.tj < tiles_j;
 }
-inline int64_t ray_grid(int n_slots, int tiles_i, int tiles_j) {
+inline int64_t ray_grid(int n_slots, int tiles_i, int tiles_j, bool pairs = false) {
+    if (pairs) return ((int64_t)tiles_i * ((tiles_j + 1) / 2) + 7) / 8 * 16 * n_slots;
     if (ray_by_columns(tiles_j)) return ((int64_t)tiles_i * tiles_j + 7) / 8 * 8 * n_slots;
     return (int64_t)n_slots * tiles_i * ((tiles_j + 7) / 8 * 8);
 }
