@@ -577,16 +577,28 @@ __host__ __device__ inline bool ray_by_pairs(int nz, int n_slots, int tiles_i, i
     return nz <= 16 && !ray_by_columns(tiles_j) &&
            (int64_t)n_slots * tiles_i * tiles_j > 2560;
 }
+// The unit of fproj_sart, which writes two outputs in that layout, as lg below. A
+// band's stores are 16 bytes of a line in each, eight XCDs sharing the line; large
+// detectors and launches (164 MB of outputs) are dealt in blocks of 64 x 64 bins,
+// whole lines. In bands or pairs and in blocks: 1600x1200 bins, 1200x600x40 voxels, 3
+// views 159 and 151 us, 15 views 732 and 644; 2048x1664 bins, 9 views, 1400x600x12
+// 388 and 345, 1400x600x60 712 and 707; 1536x1024 bins, 1000x500x45, 25 views 1137
+// and 941; below the lines 9 views 320 and 346, 640x512 bins 25 views 178 and 244.
+__host__ __device__ inline int ray_unit_sart(int nz, int n_slots, int tiles_i, int tiles_j) {
+    const int64_t tiles = (int64_t)tiles_i * tiles_j;
+    if (tiles_j >= 128 && (tiles > 7000 || tiles * n_slots > 80000)) return 4;
+    return ray_by_pairs(nz, n_slots, tiles_i, tiles_j) ? 1 : 0;
+}
 // Tile of work-group w of a launch of ray_grid() groups; false past the last
-// unit. pairs: by ray_by_pairs, the same for both.
+// unit. lg (the same for both): 0, or units of 2^lg bands of one tile column.
 __host__ __device__ inline bool ray_tile(int w, int n_slots, int tiles_i, int tiles_j,
-                                         RayTile& t, bool pairs = false) {
-    if (pairs) {
-        const int pairs_j = (tiles_j + 1) >> 1, v = w >> 4, rest = v / n_slots;
-        const int unit = rest * 8 + (w & 7);
-        t.slot = v - rest * n_slots;
-        t.ti = unit / pairs_j;
-        t.tj = 2 * (unit - t.ti * pairs_j) + ((w >> 3) & 1);
+                                         RayTile& t, int lg = 0) {
+    if (lg) {
+        const int units_j = (tiles_j + (1 << lg) - 1) >> lg, v = w >> 3;
+        const int rest = (v >> lg) / n_slots, unit = rest * 8 + (w & 7);
+        t.slot = (v >> lg) - rest * n_slots;
+        t.ti = unit / units_j;
+        t.tj = ((unit - t.ti * units_j) << lg) + (v & ((1 << lg) - 1));
         return t.ti < tiles_i && t.tj < tiles_j;
     }
     const int u = w >> 3, rest = u / n_slots;
@@ -601,8 +613,11 @@ __host__ __device__ inline bool ray_tile(int w, int n_slots, int tiles_i, int ti
     t.tj = (rest / tiles_i) * 8 + (w & 7);
     return t.tj < tiles_j;
 }
-inline int64_t ray_grid(int n_slots, int tiles_i, int tiles_j, bool pairs = false) {
-    if (pairs) return ((int64_t)tiles_i * ((tiles_j + 1) / 2) + 7) / 8 * 16 * n_slots;
+inline int64_t ray_grid(int n_slots, int tiles_i, int tiles_j, int lg = 0) {
+    if (lg) {
+        const int64_t units = (int64_t)tiles_i * ((tiles_j + (1 << lg) - 1) >> lg);
+        return ((units + 7) / 8 * 8 * n_slots) << lg;
+    }
     if (ray_by_columns(tiles_j)) return ((int64_t)tiles_i * tiles_j + 7) / 8 * 8 * n_slots;
     return (int64_t)n_slots * tiles_i * ((tiles_j + 7) / 8 * 8);
 }

@@ -365,7 +365,6 @@ __device__ __forceinline__ float walk(const DevGeom& g, const VolReader<TI>& img
 // detector-row-major layout [slot][nby][nbx]); 4 / 5 gamma (ray length / row
 // sum) times yry(y, r) with y, r read in the reference layout and the product
 // written row-major (the fused precompute).
-constexpr bool ref_layout(int kind) { return kind != 3; }  // written or read
 // Bin (i, j) of launch slot `slot` (view parameters v).
 template <int KIND, typename TI, typename TO>
 __device__ __forceinline__ void project_bin(const DevGeom& g, const ViewTab& v, int slot, int i,
@@ -443,20 +442,25 @@ __device__ __forceinline__ bool bin_of_tile(const DevGeom& g, const RayTile& t, 
     j = t.tj * TJ + (threadIdx.x >> 6);
     return i < g.nbx && j < g.nby;
 }
-// Work-groups of a single-geometry launch, and the bin of this thread of one. REF:
-// the kernel writes or reads the reference layout.
-template <bool REF = false>
+// Work-groups of a single-geometry launch, and the bin of this thread of one. OUT:
+// how the tiles are dealt, by what the kernel writes (or reads).
+enum Dealt { ROWS, REF, REF_SART };
+template <Dealt OUT>
+__host__ __device__ __forceinline__ int unit_of(const DevGeom& g, int n_slots, int ti, int tj) {
+    if (OUT == REF_SART) return ray_unit_sart(g.nz, n_slots, ti, tj);
+    return OUT == REF && ray_by_pairs(g.nz, n_slots, ti, tj) ? 1 : 0;
+}
+template <Dealt OUT = ROWS>
 int64_t groups_of(const DevGeom& g, int n_slots) {
     const int ti = ray_tiles_i(g), tj = ray_tiles_j(g, TILE_J);
-    return ray_grid(n_slots, ti, tj, REF && ray_by_pairs(g.nz, n_slots, ti, tj));
+    return ray_grid(n_slots, ti, tj, unit_of<OUT>(g, n_slots, ti, tj));
 }
-template <bool REF = false>
+template <Dealt OUT = ROWS>
 __device__ __forceinline__ bool bin_of_group(const DevGeom& g, int n_slots, int& slot, int& i,
                                              int& j) {
     const int ti = ray_tiles_i(g), tj = ray_tiles_j(g, TILE_J);
     RayTile t;
-    if (!ray_tile(blockIdx.x, n_slots, ti, tj, t, REF && ray_by_pairs(g.nz, n_slots, ti, tj)))
-        return false;
+    if (!ray_tile(blockIdx.x, n_slots, ti, tj, t, unit_of<OUT>(g, n_slots, ti, tj))) return false;
     slot = t.slot;
     return bin_of_tile<TILE_J>(g, t, i, j);
 }
@@ -470,7 +474,7 @@ __global__ __launch_bounds__(256) void project_kernel(DevGeom g, const ViewTab* 
                                                       const float* __restrict__ b,
                                                       const float* __restrict__ r) {
     int slot, i, j;
-    if (!bin_of_group<ref_layout(KIND)>(g, n_slots, slot, i, j)) return;
+    if (!bin_of_group<KIND == 3 ? ROWS : REF>(g, n_slots, slot, i, j)) return;
     project_bin<KIND, TI, TO>(g, views[a0 + slot], slot, i, j, cos_weight, img, out, y, b, r);
 }
 
@@ -492,7 +496,7 @@ __global__ __launch_bounds__(256) void sart_project_kernel(DevGeom g,
                                                            float* __restrict__ norm,
                                                            const float* __restrict__ p_rows) {
     int slot, i, j;
-    if (!bin_of_group<!DIFF>(g, n_slots, slot, i, j)) return;
+    if (!bin_of_group<DIFF ? ROWS : REF_SART>(g, n_slots, slot, i, j)) return;
     const ViewTab v = views[a0 + slot];
     const float ex = bin_centre(g.x_d0, i, g.dbx);
     const float ey = bin_centre(g.y_d0, j, g.dby);
@@ -619,7 +623,7 @@ hipError_t launch_kind(const DevGeom& g, const ViewTab* views, int a0, int a1, i
                        const void* img, void* out, const float* y, const float* b,
                        const float* r, hipStream_t st) {
     const int n_slots = a1 - a0;
-    const int64_t nblocks = groups_of<ref_layout(KIND)>(g, n_slots);
+    const int64_t nblocks = groups_of<KIND == 3 ? ROWS : REF>(g, n_slots);
     if (nblocks == 0) return hipSuccess;
     if (nblocks > 0x7fffffff) return hipErrorInvalidValue;
     hipLaunchKernelGGL((project_kernel<KIND, TI, TO>), dim3((unsigned)nblocks), dim3(256), 0, st,
@@ -726,7 +730,7 @@ hipError_t launch_sart_project(const DevGeom& g, const ViewTab* views, int a0, i
                                int cos_weight, const float* img, float* prj, float* norm,
                                hipStream_t st) {
     const int n_slots = a1 - a0;
-    const int64_t nblocks = groups_of<true>(g, n_slots);
+    const int64_t nblocks = groups_of<REF_SART>(g, n_slots);
     if (nblocks == 0) return hipSuccess;
     if (nblocks > 0x7fffffff) return hipErrorInvalidValue;
     hipLaunchKernelGGL(sart_project_kernel<false>, dim3((unsigned)nblocks), dim3(256), 0, st, g,
