@@ -10,8 +10,9 @@
 // MI355X mapping: one ray per lane, 64 lanes along detector x (the direction
 // that is contiguous in the volume, so gathers of a wave fall in a few cache
 // lines); a work-group is a 64 x 4 bin tile of one view slot; rows of tiles of
-// all views are dealt round-robin to the XCDs (ray_tile), so each XCD gets an
-// even share of the rays through the volume and the views share its L2.
+// all views are dealt round-robin to the XCDs (ray_tile; other units where
+// ray_by_columns, ray_by_pairs or ray_unit_sart say so), so each XCD gets an even
+// share of the rays through the volume and the views share its L2.
 // Per-view trig comes from the handle's table (host FP64, rounded to float).
 // The relative stop test (lmax - at)/lmax > 1e-6 is replaced by `at < thr`
 // with thr computed once per ray as the exact float boundary of that test, so
